@@ -1284,7 +1284,7 @@ void buildContext(spg_vbd_ctx &c, const spg_vbd_object *objs, int32_t nObjects)
     c.xt.upload(hpos, c.stream);
     c.xold.upload(hzero, c.stream);
     c.mass.upload(hmass, c.stream);
-    c.counters.upload(std::vector<unsigned long long>(2, 0ull), c.stream);
+    c.counters.upload(std::vector<unsigned long long>(kCounterCells * kCounterStride, 0ull), c.stream);
     c.r2.alloc(c.nv);
     c.norms.alloc(nObjects);
     c.normsAux.alloc(nObjects);
@@ -2102,12 +2102,18 @@ int spg_vbd_get_stats(const spg_vbd_ctx *ctx, spg_vbd_stats *stats)
         if (!ctx || !stats) throw VbdError(SPG_VBD_ERR_INVALID, "null argument");
         hipCheck(hipSetDevice(c->device), "hipSetDevice");
         c->drainEvents();
-        unsigned long long cnt[2] = {0, 0};
-        hipCheck(hipMemcpyAsync(cnt, c->counters.p, sizeof(cnt), hipMemcpyDeviceToHost, c->stream), "download");
+        std::vector<unsigned long long> cells(kCounterCells * kCounterStride);
+        hipCheck(hipMemcpyAsync(cells.data(), c->counters.p, cells.size() * sizeof(cells[0]), hipMemcpyDeviceToHost,
+                                c->stream),
+                 "download");
         hipCheck(hipStreamSynchronize(c->stream), "hipStreamSynchronize");
         *stats = c->stats;
-        stats->fp64_fallbacks = static_cast<int64_t>(cnt[0]);
-        stats->skipped_blocks = static_cast<int64_t>(cnt[1]);
+        stats->fp64_fallbacks = 0;
+        stats->skipped_blocks = 0;
+        for (int k = 0; k < kCounterCells; ++k) {
+            stats->fp64_fallbacks += static_cast<int64_t>(cells[k * kCounterStride]);
+            stats->skipped_blocks += static_cast<int64_t>(cells[k * kCounterStride + 1]);
+        }
         stats->prediction_fallbacks = c->predictionFallbacks;
     });
 }
@@ -2120,8 +2126,10 @@ int spg_vbd_reset_stats(spg_vbd_ctx *ctx)
         ctx->drainEvents();
         ctx->stats = spg_vbd_stats{};
         ctx->predictionFallbacks = 0;
-        const unsigned long long zero[2] = {0, 0};
-        hipCheck(hipMemcpyAsync(ctx->counters.p, zero, sizeof(zero), hipMemcpyHostToDevice, ctx->stream), "upload");
+        const std::vector<unsigned long long> zero(kCounterCells * kCounterStride, 0ull);
+        hipCheck(hipMemcpyAsync(ctx->counters.p, zero.data(), zero.size() * sizeof(zero[0]), hipMemcpyHostToDevice,
+                                ctx->stream),
+                 "upload");
         hipCheck(hipStreamSynchronize(ctx->stream), "hipStreamSynchronize");
     });
 }

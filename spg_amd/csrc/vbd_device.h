@@ -76,6 +76,15 @@ struct NbHinge {
 };
 static_assert(sizeof(NbHinge) == 12, "hinge records are 12 bytes");
 
+// The solve's FP64-fallback and skip counts: a workgroup adds to cell blockIdx % kCounterCells, each cell a
+// 64-byte line of its own, and the host sums the cells. Atomics on one address are served one after the other,
+// about 12 ns each: with a single pair of counters a sweep in which every block takes the FP64 solve (a flat
+// cloth: the out-of-plane stiffness is only the inertia's) was bound by them, 85 us a launch on a 512x512 cloth at
+// 6 lanes per vertex and 201 us at 16. With the cells a 20-sweep step of that cloth, read back, went from 3.30 to
+// 1.92 ms; a cloth or solid without fallbacks takes the same time as before.
+constexpr int kCounterCells = 256;
+constexpr int kCounterStride = 8;
+
 struct SolveArgs {
     float4 *pos;
     const float4 *xt;
@@ -119,7 +128,7 @@ struct SolveArgs {
     const int4 *xrV[kXCls];
     const float4 *xrP[kXCls];
     int64_t xrPlane[kXCls];
-    unsigned long long *counters;  // [0] FP64 fallbacks, [1] skipped blocks
+    unsigned long long *counters;  // kCounterCells cells of kCounterStride: [0] FP64 fallbacks, [1] skipped blocks
     int32_t begin, end;            // slot range of the colour
     float invdt2;
     // neighbourhood layout (lds_staging 2): per vertex slot a row of nbW slots (entry 0 the vertex itself, then

@@ -186,8 +186,9 @@ __device__ __forceinline__ void finishVertex(const SolveArgs &a, bool active, in
     }
     const unsigned long long fb = __ballot(path == kSolvedFp64), sk = __ballot(path == kSkipped);
     if (lane64 == 0) {
-        if (fb) atomicAdd(&a.counters[0], static_cast<unsigned long long>(__popcll(fb)));
-        if (sk) atomicAdd(&a.counters[1], static_cast<unsigned long long>(__popcll(sk)));
+        unsigned long long *cell = a.counters + (blockIdx.x % kCounterCells) * kCounterStride;
+        if (fb) atomicAdd(&cell[0], static_cast<unsigned long long>(__popcll(fb)));
+        if (sk) atomicAdd(&cell[1], static_cast<unsigned long long>(__popcll(sk)));
     }
 }
 

@@ -510,3 +510,18 @@ def test_zero_mass_particles_match_oracle(oracle_threads):
     ctx.step(s.dt, 1, s.iterations, s.gravity)
     o.step(s.dt, 1, s.iterations, s.gravity)
     assert rel_err(ctx.state()[0], o.state()[0]) < 1e-5
+
+
+@pytest.mark.parametrize("lanes,block,staged", [(1, 64, 0), (6, 64, 2), (16, 64, 2), (16, 256, 0)])
+def test_fp64_solve_counts_do_not_depend_on_the_launch(lanes, block, staged):
+    """A flat cloth whose bending is far stiffer than its membrane: every block but the anchored ones has a condition
+    beyond the FP32 solve's limit (in-plane stiffness about Y t, out of plane 6 k / edge^2), whatever the launch
+    shape and number of workgroups (more than the counter cells at 16 lanes)."""
+    s = scenes.cloth(96, young=1e4, bending=1.0, pin="top_row", noise=0.0, iterations=2)
+    ctx = gpu_context(s, lanes_per_vertex=lanes, block_size=block, lds_staging=staged)
+    ctx.reset_stats()
+    ctx.step(s.dt, 1, s.iterations, s.gravity)
+    assert ctx.stats()["fp64_fallbacks"] == (s.n - s.meta["pins"]) * s.iterations
+    assert ctx.stats()["skipped_blocks"] == 0
+    ctx.reset_stats()
+    assert ctx.stats()["fp64_fallbacks"] == 0
