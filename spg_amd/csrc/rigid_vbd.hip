@@ -24,6 +24,7 @@
 #include "host_util.h"
 #include "rigid_element.h"
 #include "spg_rigid.h"
+#include "state_io.h"
 #include "vbd_device.h"
 
 using namespace spgvbd;
@@ -309,6 +310,8 @@ struct spg_rigid_ctx {
     int32_t nColors = 0;
     std::vector<int64_t> groupOffset;        // bodies of group g: [groupOffset[g], groupOffset[g + 1]) in input order
     std::vector<int64_t> slotOf;             // input body index (over all groups) -> slot
+    DevBuf<int32_t> order;                   // the same on the device
+    StateReader reader;
     std::vector<std::vector<int32_t>> colors;  // per group, per body
     std::vector<int64_t> colorStart;         // slot range of colour c: [colorStart[c], colorStart[c + 1])
     int64_t incEntries = 0, solveBytes = 0;
@@ -461,6 +464,9 @@ void buildContext(spg_rigid_ctx &c, const spg_rigid_group *groups, int32_t nGrou
         for (int32_t g = 0; g < nGroups; ++g)
             for (int64_t i = 0; i < groups[g].n_bodies; ++i) c.slotOf[c.groupOffset[g] + i] = next[c.colors[g][i]]++;
     }
+    c.order.upload(std::vector<int32_t>(c.slotOf.begin(), c.slotOf.end()), c.stream);
+    hipCheck(hipStreamSynchronize(c.stream), "hipStreamSynchronize");  // the uploaded vector ends here
+    c.reader.reserve(12 * sizeof(double), largestRange(c.groupOffset));
     // per-slot host arrays
     const int64_t nb = c.nb;
     std::vector<double> hpose(kPose * nb), hv(3 * nb, 0.0), hw(3 * nb, 0.0), hth(3 * nb), hm(nb), hIl(9 * nb),
@@ -702,20 +708,8 @@ int spg_rigid_get_state(spg_rigid_ctx *ctx, int32_t group, double *x, double *th
         hipCheck(hipSetDevice(ctx->device), "hipSetDevice");
         const int64_t b0 = ctx->groupOffset[group], n = ctx->groupOffset[group + 1] - b0;
         if (n == 0) return;
-        // fetch(src, width, offset, dst): 3 doubles at `offset` of each width-double slot record
-        auto fetch = [&](const DevBuf<double> &src, int width, int offset, double *dst) {
-            if (!dst) return;
-            std::vector<double> buf(width * ctx->nb);
-            hipCheck(hipMemcpyAsync(buf.data(), src.p, buf.size() * sizeof(double), hipMemcpyDeviceToHost, ctx->stream),
-                     "download");
-            hipCheck(hipStreamSynchronize(ctx->stream), "hipStreamSynchronize");
-            for (int64_t i = 0; i < n; ++i)
-                for (int d = 0; d < 3; ++d) dst[3 * i + d] = buf[width * ctx->slotOf[b0 + i] + offset + d];
-        };
-        fetch(ctx->pose, kPose, 0, x);
-        fetch(ctx->th, 3, 0, theta);
-        fetch(ctx->v, 3, 0, v);
-        fetch(ctx->w, 3, 0, omega);
+        const Field3<double> f[4] = {{ctx->pose.p, kPose, x}, {ctx->th.p, 3, theta}, {ctx->v.p, 3, v}, {ctx->w.p, 3, omega}};
+        ctx->reader.read(f, 4, ctx->order.p + b0, n, ctx->stream);
     });
 }
 

@@ -22,6 +22,7 @@
 #include "implicit_element.h"
 #include "host_util.h"
 #include "mlp_device.h"
+#include "state_io.h"
 
 using namespace spgvbd;
 
@@ -141,6 +142,7 @@ struct spg_vbd_ctx {
     hipEvent_t evSnap[kPipe] = {}, evCheck[kPipe] = {}, evInertialCheck = nullptr;
     hipEvent_t evFeatures = nullptr, evPrediction = nullptr;  // learned start: features ready, prediction ready
     DevBuf<int32_t> objSlots;
+    StateReader reader;
     DevBuf<int64_t> objOffsets;
     // segments of the per-object residual reduction over the particle-ordered squared residuals:
     // particles segBegin[k] .. segBegin[k + 1] - 1 belong to one object; object o owns segments
@@ -1285,6 +1287,7 @@ void buildContext(spg_vbd_ctx &c, const spg_vbd_object *objs, int32_t nObjects)
     c.xold.upload(hzero, c.stream);
     c.mass.upload(hmass, c.stream);
     c.counters.upload(std::vector<unsigned long long>(kCounterCells * kCounterStride, 0ull), c.stream);
+    c.reader.reserve(6 * sizeof(float), largestRange(c.objOffset));
     c.r2.alloc(c.nv);
     c.norms.alloc(nObjects);
     c.normsAux.alloc(nObjects);
@@ -1812,26 +1815,10 @@ int spg_vbd_get_state(spg_vbd_ctx *ctx, int32_t object, double *x, double *v)
     return guarded(ctx, [&] {
         checkObject(ctx, object);
         hipCheck(hipSetDevice(ctx->device), "hipSetDevice");
-        std::vector<float4> hp(ctx->nv), hv(ctx->nv);
-        hipCheck(hipMemcpyAsync(hp.data(), ctx->pos.p, sizeof(float4) * ctx->nv, hipMemcpyDeviceToHost, ctx->stream),
-                 "download");
-        hipCheck(hipMemcpyAsync(hv.data(), ctx->vel.p, sizeof(float4) * ctx->nv, hipMemcpyDeviceToHost, ctx->stream),
-                 "download");
-        hipCheck(hipStreamSynchronize(ctx->stream), "hipStreamSynchronize");
-        const int64_t n = ctx->objOffset[object + 1] - ctx->objOffset[object];
-        for (int64_t i = 0; i < n; ++i) {
-            const int32_t s = ctx->slotOfGid[ctx->objOffset[object] + i];
-            if (x) {
-                x[3 * i] = hp[s].x;
-                x[3 * i + 1] = hp[s].y;
-                x[3 * i + 2] = hp[s].z;
-            }
-            if (v) {
-                v[3 * i] = hv[s].x;
-                v[3 * i + 1] = hv[s].y;
-                v[3 * i + 2] = hv[s].z;
-            }
-        }
+        const int64_t b = ctx->objOffset[object], n = ctx->objOffset[object + 1] - b;
+        const Field3<float> f[2] = {{reinterpret_cast<const float *>(ctx->pos.p), 4, x},
+                                    {reinterpret_cast<const float *>(ctx->vel.p), 4, v}};
+        ctx->reader.read(f, 2, ctx->objSlots.p + b, n, ctx->stream);
     });
 }
 

@@ -16,6 +16,7 @@
 #include "coloring.h"
 #include "host_util.h"
 #include "spg_xpbd.h"
+#include "state_io.h"
 #include "vbd_device.h"
 #include "xpbd_device.h"
 #include "xpbd_element.h"
@@ -89,6 +90,7 @@ struct spg_xpbd_ctx {
 
     DevBuf<float4> pos, vel, xold, snapPos, snapVel;
     bool haveSnapshot = false;
+    StateReader reader;
     DevBuf<int2> sprI;
     DevBuf<float2> sprP;
     DevBuf<int32_t> ancI;
@@ -568,6 +570,7 @@ void buildContext(spg_xpbd_ctx &c, const spg_xpbd_object *objs, int32_t nObjects
     }
     c.pos.upload(hp, c.stream);
     c.vel.upload(hv, c.stream);
+    c.reader.reserve(6 * sizeof(float), largestRange(c.objOffset));
     c.xold.alloc(c.nv);
     c.counters.alloc(1);
     hipCheck(hipMemsetAsync(c.counters.p, 0, sizeof(unsigned long long), c.stream), "memset");
@@ -698,24 +701,9 @@ int spg_xpbd_get_state(spg_xpbd_ctx *ctx, int32_t object, double *x, double *v)
         hipCheck(hipSetDevice(ctx->device), "hipSetDevice");
         const int64_t b = ctx->objOffset[object], n = ctx->objOffset[object + 1] - b;
         if (n == 0) return;
-        std::vector<float4> hp(n), hv(n);
-        hipCheck(hipMemcpyAsync(hp.data(), ctx->pos.p + b, sizeof(float4) * n, hipMemcpyDeviceToHost, ctx->stream),
-                 "download");
-        hipCheck(hipMemcpyAsync(hv.data(), ctx->vel.p + b, sizeof(float4) * n, hipMemcpyDeviceToHost, ctx->stream),
-                 "download");
-        hipCheck(hipStreamSynchronize(ctx->stream), "hipStreamSynchronize");
-        for (int64_t i = 0; i < n; ++i) {
-            if (x) {
-                x[3 * i] = hp[i].x;
-                x[3 * i + 1] = hp[i].y;
-                x[3 * i + 2] = hp[i].z;
-            }
-            if (v) {
-                v[3 * i] = hv[i].x;
-                v[3 * i + 1] = hv[i].y;
-                v[3 * i + 2] = hv[i].z;
-            }
-        }
+        const Field3<float> f[2] = {{reinterpret_cast<const float *>(ctx->pos.p + b), 4, x},
+                                    {reinterpret_cast<const float *>(ctx->vel.p + b), 4, v}};
+        ctx->reader.read(f, 2, nullptr, n, ctx->stream);
     });
 }
 
