@@ -81,9 +81,10 @@ typedef struct {
 typedef struct {
     int32_t block_size; /* threads per workgroup of the projection kernels: 64, 128 or 256 */
     int32_t use_graph;  /* 1: capture a whole step in a hipGraph and replay it */
-    int32_t group_runs; /* 1 (default): consecutive stencil groups of at most 1024 stencils (the tail colours)
-                           run in one workgroup, in order with a barrier between them, as one launch; 0: one
-                           launch per group. Same result either way. */
+    int32_t group_runs; /* 1 (default): consecutive stencil groups run in one launch where that is faster: over
+                           tiles of particles, each with the part of its neighbours it depends on; in timed steps
+                           (spg_xpbd_set_timing) the groups of at most 1024 stencils (the tail colours) in one
+                           workgroup. 0: one launch per group. Same result either way. */
 } spg_xpbd_launch;
 
 typedef struct {
@@ -115,7 +116,8 @@ int spg_xpbd_num_particles(const spg_xpbd_ctx *ctx, int32_t object, int64_t *n);
 /* Stencil groups of one energy: colours (parallel) or serial levels; group of every stencil. */
 int spg_xpbd_num_groups(const spg_xpbd_ctx *ctx, int32_t object, int32_t energy, int32_t *n);
 int spg_xpbd_get_groups(const spg_xpbd_ctx *ctx, int32_t object, int32_t energy, int32_t *group_of_stencil);
-/* Projection kernel launches per substep (all objects together), with the launch shape's group runs. */
+/* Projection kernel launches per substep of a timed step (all objects together), with the launch shape's group
+   runs. */
 int spg_xpbd_num_launches(const spg_xpbd_ctx *ctx, int32_t *n);
 
 int spg_xpbd_set_state(spg_xpbd_ctx *ctx, int32_t object, const double *x, const double *v);

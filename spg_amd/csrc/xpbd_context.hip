@@ -119,6 +119,15 @@ struct spg_xpbd_ctx {
         int32_t first, count;  // launches[first .. first + count - 1]
     };
     std::vector<Item> plan, single;  // with group runs / one launch per group
+    // the tile plan (xpbd_tiles.h): a substep's groups in a few launches; batches empty: none. Used by steps with
+    // group_runs that are not timed (timed steps launch the groups of `plan`, so that each energy type's projections
+    // can be measured).
+    std::vector<TileBatch> batches;
+    int tilesSet = 0;
+    DevBuf<TileHeader> tileHeaders;
+    DevBuf<int32_t> tileParticles;
+    DevBuf<TileSegment> tileSegments;
+    DevBuf<float4> tileRecords, spare;  // spare: third position buffer
 
     spg_xpbd_launch launch{256, 1, 1};
     bool timing = false;
@@ -216,8 +225,71 @@ struct spg_xpbd_ctx {
         eventLaunch.clear();
     }
 
+    // A step by the tile plan. Three position buffers change roles: `start` holds the substep's start (its x_old), which
+    // stays as it is during the substep; the first batch reads it (and, for the velocities, the previous substep's
+    // start) and writes a free buffer, every later batch reads the last one and writes the other free one.
+    void enqueueTiledStep(double dt, int32_t nsub, const double *g)
+    {
+        const double h = dt / nsub;
+        XpbdTileArgs a{};
+        a.particles = tileParticles.p;
+        a.segments = tileSegments.p;
+        a.records = tileRecords.p;
+        a.counters = counters.p;
+        a.invdt2 = static_cast<float>(1.0 / (h * h));
+        a.h = static_cast<float>(h);
+        a.invhPrev = static_cast<float>(1.0 / h);
+        a.hgx = static_cast<float>(h * g[0]);
+        a.hgy = static_cast<float>(h * g[1]);
+        a.hgz = static_cast<float>(h * g[2]);
+        float4 *const buffers[3] = {pos.p, xold.p, spare.p};
+        auto freeOf = [&](const float4 *used0, const float4 *used1) {
+            for (float4 *b : buffers)
+                if (b != used0 && b != used1) return b;
+            return static_cast<float4 *>(nullptr);
+        };
+        float4 *start = pos.p, *prev = nullptr;
+        for (int32_t s = 0; s < nsub; ++s) {
+            float4 *cur = nullptr;
+            for (const TileBatch &b : batches) {
+                const int mode = cur ? 0 : s == 0 ? 1 : 2;
+                a.in = cur ? cur : start;
+                a.prev = mode == 1 ? vel.p : prev;
+                if (b.tiles) {
+                    a.out = freeOf(start, mode == 0 ? cur : prev);
+                    a.headers = tileHeaders.p + b.headerBase;
+                    a.tiles = b.tiles;
+                    a.groups = b.groups;
+                    hipCheck(launchXpbdTiles(a, mode, tilesSet, b.maxParticles, stream), "tile launch");
+                    cur = a.out;
+                    continue;
+                }
+                if (!cur) {
+                    a.out = freeOf(start, prev);
+                    hipCheck(launchXpbdStart(a, mode, static_cast<int32_t>(nv), stream), "substep start launch");
+                    cur = a.out;
+                }
+                XpbdArgs one = args(a.invdt2);
+                one.pos = cur;
+                for (int32_t k = b.firstGroup; k < b.firstGroup + b.groups; ++k)
+                    hipCheck(launchXpbdProject(launches[k].type, one, launches[k].begin, launches[k].end,
+                                               launch.block_size, stream),
+                             "projection launch");
+            }
+            prev = start;
+            start = cur;
+        }
+        hipCheck(launchXpbdEnd(start, prev, vel.p, static_cast<int32_t>(nv), a.invhPrev, stream,
+                               start == pos.p ? nullptr : pos.p),
+                 "end launch");
+    }
+
     void enqueueStep(double dt, int32_t nsub, const double *g, bool timed)
     {
+        if (launch.group_runs && !timed && !batches.empty()) {
+            enqueueTiledStep(dt, nsub, g);
+            return;
+        }
         const double h = dt / nsub;  // xpbd.cpp:22
         const float fh = static_cast<float>(h), invh = static_cast<float>(1.0 / h);
         const float hg[3] = {static_cast<float>(h * g[0]), static_cast<float>(h * g[1]), static_cast<float>(h * g[2])};
@@ -368,6 +440,41 @@ void validateEnergy(const spg_xpbd_energy &e, int64_t np)
                 throw VbdError(SPG_VBD_ERR_INVALID, "Invalid restTheta");
         }
         }
+    }
+}
+
+// Builds the tile plan and its records; without memory for them the context steps group by group.
+void buildTiles(spg_xpbd_ctx &c, const std::vector<float4> &x, const std::vector<TileGroup> &groups,
+                const std::function<void(int32_t, int32_t *)> &stencils)
+{
+    try {
+        for (const auto &g : groups) c.tilesSet = std::max(c.tilesSet, tileSet(g.type));
+        const TilePlan plan = buildTilePlan(x.empty() ? nullptr : &x[0].x, 4, c.objOffset, groups, stencils, tileThreads(c.tilesSet));
+        if (plan.batches.empty()) return;
+        DevBuf<TileEntry> entries;
+        DevBuf<int64_t> segmentEntry;
+        c.tileHeaders.upload(plan.headers, c.stream);
+        c.tileParticles.upload(plan.particles, c.stream);
+        c.tileSegments.upload(plan.segments, c.stream);
+        c.tileRecords.alloc(plan.recordSize);
+        c.spare.alloc(c.nv);
+        entries.upload(plan.entries, c.stream);
+        segmentEntry.upload(plan.segmentEntry, c.stream);
+        hipCheck(launchTileRecords(c.args(0.f), c.tileSegments.p, static_cast<int32_t>(plan.segments.size()),
+                                   segmentEntry.p, entries.p, c.tileRecords.p, c.stream),
+                 "tile records launch");
+        hipCheck(hipStreamSynchronize(c.stream), "hipStreamSynchronize");
+        c.batches = plan.batches;
+    } catch (const std::bad_alloc &) {
+    } catch (const VbdError &) {
+        (void)hipGetLastError();
+    }
+    if (c.batches.empty()) {
+        c.tileHeaders.release();
+        c.tileParticles.release();
+        c.tileSegments.release();
+        c.tileRecords.release();
+        c.spare.release();
     }
 }
 
@@ -574,6 +681,16 @@ void buildContext(spg_xpbd_ctx &c, const spg_xpbd_object *objs, int32_t nObjects
     c.xold.alloc(c.nv);
     c.counters.alloc(1);
     hipCheck(hipMemsetAsync(c.counters.p, 0, sizeof(unsigned long long), c.stream), "memset");
+
+    std::vector<TileGroup> groups;
+    for (const auto &L : c.launches) groups.push_back({L.type, stencilSizeOf(L.type), L.end - L.begin, L.begin});
+    buildTiles(c, hp, groups, [&](int32_t g, int32_t *out) {
+        const auto &L = c.launches[g];
+        const int ss = stencilSizeOf(L.type);
+        const int32_t off = L.type >= SPG_VBD_SPRING_CONTINUUM ? extBase[L.type] : 0;
+        for (int32_t i = L.begin; i < L.end; ++i)
+            for (int d = 0; d < ss; ++d) *out++ = gidx(ent[L.type][i - off], d);
+    });
     hipCheck(hipStreamSynchronize(c.stream), "hipStreamSynchronize");
 }
 

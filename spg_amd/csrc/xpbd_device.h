@@ -19,6 +19,8 @@
 
 #include <cstdint>
 
+#include "xpbd_tiles.h"
+
 namespace spgvbd {
 
 struct XpbdArgs {
@@ -75,8 +77,30 @@ hipError_t launchXpbdBegin(float4 *pos, float4 *vel, float4 *xold, int32_t n, fl
                            hipStream_t stream);
 hipError_t launchXpbdBoundary(float4 *pos, float4 *xold, int32_t n, float invhPrev, float h, float gx, float gy,
                               float gz, hipStream_t stream);
+// copy: where not null, x is written there too.
 hipError_t launchXpbdEnd(const float4 *pos, const float4 *xold, float4 *vel, int32_t n, float invh,
-                         hipStream_t stream);
+                         hipStream_t stream, float4 *copy = nullptr);
+
+// One batch of a tile plan (xpbd_tiles.h). start 1 / 2: the batch begins a substep, and reads its particles at the
+// substep's start from `in` and `prev` (the velocities in the first substep of a step, else the positions one substep
+// earlier); 0: `in` as it is. `out` is another buffer than `in` and `prev`.
+struct XpbdTileArgs {
+    const float4 *in, *prev;
+    float4 *out;
+    const TileHeader *headers;
+    const int32_t *particles;
+    const TileSegment *segments;
+    const float4 *records;
+    unsigned long long *counters;
+    int32_t tiles, groups;
+    float invdt2, h, invhPrev, hgx, hgy, hgz;
+};
+hipError_t launchXpbdTiles(const XpbdTileArgs &a, int start, int set, int32_t maxParticles, hipStream_t stream);
+// The particles at a substep's start (start 1 or 2), where its first group runs alone.
+hipError_t launchXpbdStart(const XpbdTileArgs &a, int start, int32_t n, hipStream_t stream);
+// Writes the tile records of a plan from the stencils' records.
+hipError_t launchTileRecords(const XpbdArgs &a, const TileSegment *segments, int32_t nSegments,
+                             const int64_t *segmentEntry, const TileEntry *entries, float4 *records, hipStream_t stream);
 // Check hook: n independent projections of one type from FP64 inputs (xs: n * size * 3, w: n * size,
 // params in the C-ABI layout), computed in float (precision 0) or double (1); dx: n * size * 3.
 hipError_t launchXpbdProjectCheck(int type, int64_t n, const double *xs, const double *w, const double *params,
