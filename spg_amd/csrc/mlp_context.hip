@@ -33,8 +33,6 @@ uint64_t splitmix64(uint64_t &s)
 }
 double uniform01(uint64_t &s) { return static_cast<double>(splitmix64(s) >> 11) * (1.0 / 9007199254740992.0); }
 
-int64_t roundUp(int64_t n, int64_t m) { return (n + m - 1) / m * m; }
-
 }  // namespace
 
 struct spg_mlp {
@@ -44,18 +42,16 @@ struct spg_mlp {
 
     int64_t wOff[kMlpLayers]{}, bOff[kMlpLayers]{}, total = 0;  // padded master layout
     DevBuf<float> P, G, M, V;                                   // parameters, gradients, Adam moments
-    DevBuf<__bf16> wb[kMlpLayers], wtb[kMlpLayers];              // BF16 W (out x in) and W^T (in x out)
     DevBuf<float> mean, invStd;
-    DevBuf<unsigned char> frag;  // weights in the fused inference kernel's operand order
+    DevBuf<unsigned char> frag;  // weights in the kernels' operand order
     int maxBlocks = 512;         // persistent workgroups of the fused inference kernel
     std::vector<float> hMean, hStd;
     int64_t adamT = 0;
     int32_t historyBase = 0;  // 1: the output is the change of the previous substep's offset (see spg_mlp_set_history_base)
 
     // workspaces
-    int64_t trainRows = 0;
-    DevBuf<__bf16> X, XT, H[2], HT[3], dY, dYT, dZb[2], dZT;
-    DevBuf<float> T, Z[3], Yf, dYf, dZf;
+    DevBuf<float> partial;
+    DevBuf<double> lossPartial;
     DevBuf<double> loss;
     DevBuf<int32_t> index;
     DevBuf<float> dataF, dataT;
@@ -79,10 +75,7 @@ struct spg_mlp {
         G.alloc(total);
         M.alloc(total);
         V.alloc(total);
-        for (int l = 0; l < kMlpLayers; ++l) {
-            wb[l].alloc(static_cast<size_t>(kLayerOut[l]) * kLayerIn[l]);
-            wtb[l].alloc(static_cast<size_t>(kLayerOut[l]) * kLayerIn[l]);
-        }
+        loss.alloc(1);
         mean.alloc(kMlpFeatures);
         invStd.alloc(kMlpFeatures);
         frag.alloc(mlpFragBytes());
@@ -153,109 +146,49 @@ struct spg_mlp {
         hipCheck(hipStreamSynchronize(stream), "hipStreamSynchronize");
     }
 
-    void refreshWeights()
-    {
-        for (int l = 0; l < kMlpLayers; ++l)
-            hipCheck(launchWeightCopies(P.p + wOff[l], kLayerOut[l], kLayerIn[l], wb[l].p, wtb[l].p, stream),
-                     "weight copies");
-        hipCheck(launchMlpFrag(P.p + wOff[0], P.p + wOff[1], P.p + wOff[2], P.p + wOff[3], frag.p, stream),
-                 "fragment launch");
-    }
+    void refreshWeights() { hipCheck(launchMlpFrag(P.p, frag.p, stream), "fragment launch"); }
 
-    void reserveTrain(int64_t rows)
+    // One batch of n rows (through `index`, or the first n without one): its gradient into G, or an Adam step with
+    // learning rate lr; adds its squared error to the loss.
+    void batch(const int32_t *index, int n, bool adam, float lr)
     {
-        if (rows <= trainRows) return;
-        X.alloc(rows * kMlpIn);
-        XT.alloc(rows * kMlpIn);
-        T.alloc(rows * kMlpOut);
-        for (int i = 0; i < 2; ++i) H[i].alloc(rows * kMlpHidden);
-        for (int i = 0; i < 3; ++i) {
-            HT[i].alloc(rows * kMlpHidden);
-            Z[i].alloc(rows * kMlpHidden);
+        // a workgroup per row block up to one per compute unit, then several row blocks each
+        const int blocks = mlpTrainBlocks(n), parts = std::min(blocks, std::max(1, maxBlocks / 2));
+        partial.reserve(static_cast<size_t>(parts) * kMlpPadded);
+        lossPartial.reserve(parts);
+        MlpTrainArgs t{};
+        t.features = dataF.p;
+        t.targets = dataT.p;
+        t.index = index;
+        t.mean = mean.p;
+        t.invStd = invStd.p;
+        t.params = P.p;
+        t.frag = frag.p;
+        t.n = n;
+        t.rowBlocks = blocks;
+        t.partial = partial.p;
+        t.lossPartial = lossPartial.p;
+        hipCheck(launchMlpTrain(t, parts, stream), "gradient launch");
+        MlpUpdateArgs u{};
+        u.partial = partial.p;
+        u.lossPartial = lossPartial.p;
+        u.parts = parts;
+        u.loss = loss.p;
+        u.grad = G.p;
+        if (adam) {
+            adamT += 1;
+            u.params = P.p;
+            u.m = M.p;
+            u.v = V.p;
+            u.frag = frag.p;
+            u.lr = lr;
+            u.b1 = 0.9f;
+            u.b2 = 0.999f;
+            u.eps = 1e-8f;
+            u.c1 = 1.f - powf(u.b1, static_cast<float>(adamT));
+            u.c2 = 1.f - powf(u.b2, static_cast<float>(adamT));
         }
-        Yf.alloc(rows * kMlpInferCols);
-        dYf.alloc(rows * kMlpOutPad);
-        dY.alloc(rows * kMlpOutPad);
-        dYT.alloc(rows * kMlpOutPad);
-        for (int i = 0; i < 2; ++i) dZb[i].alloc(rows * kMlpHidden);
-        dZT.alloc(rows * kMlpHidden);
-        dZf.alloc(rows * kMlpHidden);
-        loss.alloc(1);
-        trainRows = rows;
-    }
-
-    void gemm(const __bf16 *A, int lda, const __bf16 *B, int ldb, int64_t Mr, int N, int K, const GemmEpilogue &ep)
-    {
-        hipCheck(launchGemmNT(A, lda, B, ldb, static_cast<int>(Mr), N, K, ep, stream), "gemm launch");
-    }
-
-    // Forward pass over `rows` packed rows in X; y (FP32, stride ldy >= 16) receives the outputs. With
-    // `train`, keeps Z (pre-activations) and transposed activations for the backward pass.
-    void forward(int64_t rows, bool train, float *y, int ldy)
-    {
-        const __bf16 *A = X.p;
-        int lda = kMlpIn;
-        for (int l = 0; l < 3; ++l) {
-            GemmEpilogue ep;
-            ep.bias = P.p + bOff[l];
-            ep.act = 1;
-            ep.hOut = H[l & 1].p;
-            ep.ldh = kMlpHidden;
-            if (train) {
-                ep.zOut = Z[l].p;
-                ep.ldz = kMlpHidden;
-                ep.hTOut = HT[l].p;
-                ep.ldht = static_cast<int>(rows);
-            }
-            gemm(A, lda, wb[l].p, kLayerIn[l], rows, kMlpHidden, kLayerIn[l], ep);
-            A = H[l & 1].p;
-            lda = kMlpHidden;
-        }
-        GemmEpilogue ep;
-        ep.bias = P.p + bOff[3];
-        ep.zOut = y;
-        ep.ldz = ldy;
-        gemm(A, lda, wb[3].p, kMlpHidden, rows, kMlpInferCols, kMlpHidden, ep);
-    }
-
-    // Gradient of the batch loss into G, given the forward pass of `rows` rows (n real) and targets T.
-    void backward(int64_t rows, int n)
-    {
-        const int r = static_cast<int>(rows);
-        hipCheck(launchLossGrad(Yf.p, kMlpInferCols, T.p, kMlpOut, n, r, kMlpOutPad, dYf.p, dY.p, dYT.p, loss.p, stream),
-                 "loss launch");
-        GemmEpilogue e;
-        // layer 4: dW4 = dY^T H3, db4 = colsum dY
-        e.zOut = G.p + wOff[3];
-        e.ldz = kMlpHidden;
-        gemm(dYT.p, r, HT[2].p, r, kMlpOutPad, kMlpHidden, r, e);
-        hipCheck(launchColSum(dYf.p, kMlpOutPad, r, kMlpOutPad, G.p + bOff[3], stream), "colsum");
-        // dZ3 = (dY W4) . silu'(Z3)
-        const __bf16 *dIn = dY.p;
-        int ldIn = kMlpOutPad, kIn = kMlpOutPad;
-        for (int l = 2; l >= 0; --l) {
-            GemmEpilogue d;
-            d.dactZ = Z[l].p;
-            d.lddz = kMlpHidden;
-            d.zOut = dZf.p;
-            d.ldz = kMlpHidden;
-            if (l > 0) {
-                d.hOut = dZb[l & 1].p;
-                d.ldh = kMlpHidden;
-            }
-            d.hTOut = dZT.p;
-            d.ldht = r;
-            gemm(dIn, ldIn, wtb[l + 1].p, kLayerOut[l + 1], rows, kMlpHidden, kIn, d);
-            // dW_l = dZ_l^T H_{l-1} (X for the first layer), db_l = colsum dZ_l
-            GemmEpilogue w;
-            w.zOut = G.p + wOff[l];
-            w.ldz = kLayerIn[l];
-            gemm(dZT.p, r, l > 0 ? HT[l - 1].p : XT.p, r, kMlpHidden, kLayerIn[l], r, w);
-            hipCheck(launchColSum(dZf.p, kMlpHidden, r, kMlpHidden, G.p + bOff[l], stream), "colsum");
-            dIn = dZb[l & 1].p;
-            ldIn = kMlpHidden;
-            kIn = kMlpHidden;
-        }
+        hipCheck(launchMlpUpdate(u, adam, stream), "update launch");
     }
 
     // Fused inference on device features (n x 24) into y (stride ldy >= 3), ordered on the caller's
@@ -444,20 +377,14 @@ int spg_mlp_loss_grad(spg_mlp *net, const float *features, const float *targets,
         if (n <= 0 || n > SPG_MLP_MAX_GRAD_ROWS) throw VbdError(SPG_VBD_ERR_INVALID, "row count out of range");
         requireFinite(features, n * kMlpFeatures, "features");
         requireFinite(targets, n * kMlpOut, "targets");
-        const int64_t rows = roundUp(n, 64);
-        net->reserveTrain(rows);
         hipStream_t s = net->stream;
         net->dataF.reserve(n * kMlpFeatures);
         net->dataT.reserve(n * kMlpOut);
         hipCheck(hipMemcpyAsync(net->dataF.p, features, sizeof(float) * n * kMlpFeatures, hipMemcpyHostToDevice, s),
                  "upload");
         hipCheck(hipMemcpyAsync(net->dataT.p, targets, sizeof(float) * n * kMlpOut, hipMemcpyHostToDevice, s), "upload");
-        hipCheck(launchPackInput(net->dataF.p, net->dataT.p, nullptr, net->mean.p, net->invStd.p, static_cast<int>(n),
-                                 static_cast<int>(rows), net->X.p, net->XT.p, net->T.p, s),
-                 "pack launch");
         hipCheck(hipMemsetAsync(net->loss.p, 0, sizeof(double), s), "memset");
-        net->forward(rows, true, net->Yf.p, kMlpInferCols);
-        net->backward(rows, static_cast<int>(n));
+        net->batch(nullptr, static_cast<int>(n), false, 0.f);
         double se = 0.0;
         hipCheck(hipMemcpyAsync(&se, net->loss.p, sizeof(double), hipMemcpyDeviceToHost, s), "download");
         const auto flat = net->downloadFlat(net->G.p);  // synchronises
@@ -493,7 +420,6 @@ int spg_mlp_train(spg_mlp *net, const float *features, const float *targets, int
             net->setNormalization(m.data(), sd.data());
         }
         hipStream_t s = net->stream;
-        net->reserveTrain(batch);
         net->dataF.reserve(n * kMlpFeatures);
         net->dataT.reserve(n * kMlpOut);
         net->index.reserve(n);
@@ -516,18 +442,9 @@ int spg_mlp_train(spg_mlp *net, const float *features, const float *targets, int
             for (int64_t b = 0; b < perEpoch; ++b, ++stepNo) {
                 const int64_t r0 = b * batch;
                 const int cnt = static_cast<int>(std::min<int64_t>(batch, n - r0));
-                hipCheck(launchPackInput(net->dataF.p, net->dataT.p, net->index.p + r0, net->mean.p, net->invStd.p, cnt,
-                                         batch, net->X.p, net->XT.p, net->T.p, s),
-                         "pack launch");
-                net->forward(batch, true, net->Yf.p, kMlpInferCols);
-                net->backward(batch, cnt);
                 const double frac = totalSteps > 1 ? static_cast<double>(stepNo) / (totalSteps - 1) : 0.0;
                 const float lrNow = static_cast<float>(lr * (0.05 + 0.95 * 0.5 * (1.0 + std::cos(3.14159265358979323846 * frac))));
-                net->adamT += 1;
-                hipCheck(launchAdam(net->P.p, net->G.p, net->M.p, net->V.p, net->total, lrNow, 0.9f, 0.999f, 1e-8f,
-                                    net->adamT, s),
-                         "adam launch");
-                net->refreshWeights();
+                net->batch(net->index.p + r0, cnt, true, lrNow);
             }
             double se = 0.0;
             hipCheck(hipMemcpyAsync(&se, net->loss.p, sizeof(double), hipMemcpyDeviceToHost, s), "download");

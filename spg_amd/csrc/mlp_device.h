@@ -16,40 +16,42 @@ constexpr int kMlpOut = 3;
 constexpr int kMlpOutPad = 32;  // output rows of the last weight padded to one MFMA K step
 constexpr int kMlpLayers = 4;
 
-// What the GEMM does with an accumulator tile C[row][col] before storing it:
-//   v = C; if dactZ: v *= silu'(dactZ[row][col]); if bias: v += bias[col];
-//   zOut[row][col] = v (FP32); h = act ? silu(v) : v; hOut[row][col] = bf16(h); hTOut[col][row] = bf16(h).
-struct GemmEpilogue {
-    const float *bias = nullptr;
-    int act = 0;
-    const float *dactZ = nullptr;
-    int lddz = 0;
-    float *zOut = nullptr;
-    int ldz = 0;
-    __bf16 *hOut = nullptr;
-    int ldh = 0;
-    __bf16 *hTOut = nullptr;
-    int ldht = 0;
+constexpr int kMlpPadded = kMlpHidden * (kMlpIn + 1) + 2 * kMlpHidden * (kMlpHidden + 1) + kMlpOutPad * (kMlpHidden + 1);
+
+// The gradient of one batch: rows index[0 .. n) (0 .. n without an index) of a feature table (n x 24 FP32, standardised
+// here) and its targets (n x 3), in `parts` workgroups that share the row blocks of mlpTrainBlocks(n); each leaves its
+// sums in partial (kMlpPadded floats, padded master layout) and its squared error in lossPartial.
+struct MlpTrainArgs {
+    const float *features, *targets;
+    const int32_t *index;
+    const float *mean, *invStd;
+    const float *params;  // padded master layout (the biases are read from it)
+    const void *frag;
+    int32_t n, rowBlocks;
+    float *partial;
+    double *lossPartial;
 };
+int mlpTrainBlocks(int64_t rows);
+hipError_t launchMlpTrain(const MlpTrainArgs &a, int parts, hipStream_t stream);
+// The sums over the parts: into grad, or (adam) an Adam step of the parameters, moments and fragments. Adds the batch's
+// squared error to *loss.
+struct MlpUpdateArgs {
+    const float *partial;
+    const double *lossPartial;
+    int32_t parts;
+    double *loss;
+    float *grad;
+    float *params, *m, *v;
+    void *frag;
+    float lr, b1, b2, eps, c1, c2;  // c1, c2: 1 - b1^t, 1 - b2^t
+};
+hipError_t launchMlpUpdate(const MlpUpdateArgs &a, bool adam, hipStream_t stream);
 
-// C[M x N] = A[M x K] * B[N x K]^T, bf16 operands, FP32 accumulation. M, N multiples of 16, K multiple
-// of 32, lda and ldb multiples of 8 (16-byte fragments).
-hipError_t launchGemmNT(const __bf16 *A, int lda, const __bf16 *B, int ldb, int M, int N, int K, const GemmEpilogue &ep,
-                        hipStream_t stream);
-hipError_t launchLossGrad(const float *y, int ldy, const float *t, int outs, int n, int rows, int cols, float *dYf,
-                          __bf16 *dY, __bf16 *dYT, double *loss, hipStream_t stream);
-hipError_t launchColSum(const float *m, int ld, int rows, int cols, float *out, hipStream_t stream);
-hipError_t launchAdam(float *p, const float *g, float *m, float *v, int64_t n, float lr, float b1, float b2, float eps,
-                      int64_t t, hipStream_t stream);
-hipError_t launchWeightCopies(const float *w, int rows, int cols, __bf16 *wb, __bf16 *wtb, hipStream_t stream);
-hipError_t launchPackInput(const float *f, const float *t, const int32_t *index, const float *mean, const float *invStd,
-                           int n, int rows, __bf16 *X, __bf16 *XT, float *tOut, hipStream_t stream);
-
-// Fused inference (all layers in registers, weights staged in LDS): fragments of the weights in the
-// kernel's operand order are rebuilt from the FP32 master weights by launchMlpFrag after every change.
+// The weights in the kernels' operand order, for inference and the gradient: rebuilt from the FP32 master parameters
+// (padded layout) by launchMlpFrag, kept up to date by launchMlpUpdate.
 size_t mlpFragBytes();
-hipError_t launchMlpFrag(const float *w1, const float *w2, const float *w3, const float *w4, void *frag,
-                         hipStream_t stream);
+hipError_t launchMlpFrag(const float *params, void *frag, hipStream_t stream);
+// Fused inference: all layers in registers, weights staged in LDS.
 // y[row][0..2] = network(f[row]) for rows < n (f: n x 24 FP32, y stride ldy >= 3); at most maxBlocks
 // persistent workgroups of 256 threads.
 hipError_t launchMlpInfer(const float *f, int n, const float *mean, const float *invStd, const void *frag,
@@ -82,8 +84,6 @@ hipError_t launchSmoothPrediction(const float *y, float *out, const int32_t *nbP
 hipError_t launchGate(float4 *pos, const float4 *xt, const int32_t *objOfSlot, const int32_t *reject, int32_t n,
                       hipStream_t stream);
 
-// Columns of the training forward pass's output buffer (the last layer is computed 16 wide).
-constexpr int kMlpInferCols = 16;
 // Network inference on device-resident features (n x kMlpFeatures FP32) into y (n rows, stride
 // ldy >= kMlpOut), ordered on `stream`, with the fused kernel. Throws VbdError. Defined with the
 // network object.

@@ -1,12 +1,10 @@
 // Kernels of the learned warm start: a per-vertex MLP (24 -> 128 -> 128 -> 128 -> 3, SiLU) with BF16
-// weights and activations on CDNA4 matrix cores (v_mfma_f32_16x16x32_bf16), FP32 accumulation.
+// weights and activations on CDNA4 matrix cores (v_mfma_f32_16x16x32_bf16), FP32 accumulation: inference, the
+// gradient of a batch (forward and backward in one kernel), and the update of the weights.
 //
-// Every GEMM of training and inference is written as C[M x N] = A[M x K] * B[N x K]^T with both operands
-// row-major and K contiguous ("NT"), so that each lane's MFMA operand fragment is one 16-byte load:
-//   forward      Z = X W      with B = W^T stored as (out x in)
-//   input grads  dX = dZ W^T  with B = W stored as (in x out)
-//   weight grads dW = X^T dZ  with A = X^T and B = dZ^T (both stored transposed by the epilogues)
-// plus the feature kernel, the loss gradient, bias gradients, Adam, and the fused inference kernel.
+// MFMA operand layout (16x16x32): lane l holds row (l % 16) of A and row (l % 16) of B at K offsets 8 (l / 16) .. +7
+// (the same K split for both operands, so the products pair up); the accumulator holds C[4 (l / 16) + r][l % 16],
+// r = 0 .. 3.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -23,166 +21,13 @@ typedef __attribute__((ext_vector_type(4))) float f32x4;
 
 __device__ __forceinline__ float sigmoidf(float z) { return 1.0f / (1.0f + __expf(-z)); }
 __device__ __forceinline__ float silu(float z) { return z * sigmoidf(z); }
-__device__ __forceinline__ float siluGrad(float z)
-{
-    const float s = sigmoidf(z);
-    return s * (1.0f + z * (1.0f - s));
-}
 
-__device__ __forceinline__ bf16x8 loadFrag(const __bf16 *p) { return *reinterpret_cast<const bf16x8 *>(p); }
 __device__ __forceinline__ bf16x8 zeroFrag()
 {
     bf16x8 z;
 #pragma unroll
     for (int i = 0; i < 8; ++i) z[i] = static_cast<__bf16>(0.0f);
     return z;
-}
-
-// One workgroup of 4 wavefronts computes a 64x64 tile; each wavefront a 32x32 quarter as 2x2 MFMA
-// blocks of 16x16. MFMA operand layout (16x16x32): lane l holds row (l % 16) of A and row (l % 16)
-// of B at K offsets 8 (l / 16) .. +7 (the same K split for both operands, so the products pair
-// up); the accumulator holds C[4 (l / 16) + r][l % 16], r = 0..3.
-// Requirements (checked by the launcher): M, N multiples of 16, K multiple of 32, lda/ldb multiples of 8.
-__global__ void __launch_bounds__(256) gemmNTKernel(const __bf16 *__restrict__ A, int lda, const __bf16 *__restrict__ B,
-                                                    int ldb, int M, int N, int K, GemmEpilogue ep)
-{
-    const int lane = threadIdx.x & 63;
-    const int wave = threadIdx.x >> 6;
-    const int m0 = blockIdx.y * 64 + (wave >> 1) * 32;
-    const int n0 = blockIdx.x * 64 + (wave & 1) * 32;
-    const int r16 = lane & 15;
-    const int kq = (lane >> 4) * 8;
-    f32x4 acc[2][2];
-#pragma unroll
-    for (int i = 0; i < 2; ++i)
-#pragma unroll
-        for (int j = 0; j < 2; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-    const bool rowOk[2] = {m0 < M, m0 + 16 < M};
-    const bool colOk[2] = {n0 < N, n0 + 16 < N};
-    for (int k0 = 0; k0 < K; k0 += 32) {
-        bf16x8 a[2], b[2];
-#pragma unroll
-        for (int i = 0; i < 2; ++i)
-            a[i] = rowOk[i] ? loadFrag(A + static_cast<int64_t>(m0 + i * 16 + r16) * lda + k0 + kq) : zeroFrag();
-#pragma unroll
-        for (int j = 0; j < 2; ++j)
-            b[j] = colOk[j] ? loadFrag(B + static_cast<int64_t>(n0 + j * 16 + r16) * ldb + k0 + kq) : zeroFrag();
-#pragma unroll
-        for (int i = 0; i < 2; ++i)
-#pragma unroll
-            for (int j = 0; j < 2; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[i], b[j], acc[i][j], 0, 0, 0);
-    }
-#pragma unroll
-    for (int i = 0; i < 2; ++i)
-#pragma unroll
-        for (int j = 0; j < 2; ++j) {
-            if (!rowOk[i] || !colOk[j]) continue;
-            const int col = n0 + j * 16 + r16;
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const int row = m0 + i * 16 + (lane >> 4) * 4 + r;
-                float v = acc[i][j][r];
-                if (ep.dactZ) v *= siluGrad(ep.dactZ[static_cast<int64_t>(row) * ep.lddz + col]);
-                if (ep.bias) v += ep.bias[col];
-                if (ep.zOut) ep.zOut[static_cast<int64_t>(row) * ep.ldz + col] = v;
-                const float h = ep.act ? silu(v) : v;
-                if (ep.hOut) ep.hOut[static_cast<int64_t>(row) * ep.ldh + col] = static_cast<__bf16>(h);
-                if (ep.hTOut) ep.hTOut[static_cast<int64_t>(col) * ep.ldht + row] = static_cast<__bf16>(h);
-            }
-        }
-}
-
-// dY = 2 (y - t) / n on the real rows and the first `outs` columns, zero elsewhere; bf16 row-major and
-// transposed copies and an FP32 copy; the squared error summed into *loss.
-__global__ void __launch_bounds__(256) lossGradKernel(const float *__restrict__ y, int ldy, const float *__restrict__ t,
-                                                      int outs, int n, int rows, int cols, float *__restrict__ dYf,
-                                                      __bf16 *__restrict__ dY, __bf16 *__restrict__ dYT,
-                                                      double *__restrict__ loss)
-{
-    const int64_t idx = blockIdx.x * static_cast<int64_t>(blockDim.x) + threadIdx.x;
-    const int64_t total = static_cast<int64_t>(rows) * cols;
-    float se = 0.f;
-    if (idx < total) {
-        const int row = static_cast<int>(idx / cols), col = static_cast<int>(idx % cols);
-        float g = 0.f;
-        if (row < n && col < outs) {
-            const float d = y[static_cast<int64_t>(row) * ldy + col] - t[static_cast<int64_t>(row) * outs + col];
-            se = d * d;
-            g = 2.0f * d / static_cast<float>(n);
-        }
-        dYf[idx] = g;
-        dY[idx] = static_cast<__bf16>(g);
-        dYT[static_cast<int64_t>(col) * rows + row] = static_cast<__bf16>(g);
-    }
-    // wavefront sum, one atomic per wavefront
-    for (int off = 32; off > 0; off >>= 1) se += __shfl_down(se, off, 64);
-    if ((threadIdx.x & 63) == 0 && se != 0.f) atomicAdd(loss, static_cast<double>(se));
-}
-
-// Column sums of a row-major FP32 matrix (bias gradients): one block per column, fixed order.
-__global__ void __launch_bounds__(256) colSumKernel(const float *__restrict__ m, int ld, int rows, float *__restrict__ out)
-{
-    __shared__ float part[256];
-    const int col = blockIdx.x;
-    float s = 0.f;
-    for (int r = threadIdx.x; r < rows; r += blockDim.x) s += m[static_cast<int64_t>(r) * ld + col];
-    part[threadIdx.x] = s;
-    __syncthreads();
-    for (int w = 128; w > 0; w >>= 1) {
-        if (threadIdx.x < w) part[threadIdx.x] += part[threadIdx.x + w];
-        __syncthreads();
-    }
-    if (threadIdx.x == 0) out[col] = part[0];
-}
-
-// Adam (Kingma & Ba 2015) on FP32 master parameters.
-__global__ void __launch_bounds__(256) adamKernel(float *__restrict__ p, const float *__restrict__ g, float *__restrict__ m,
-                                                  float *__restrict__ v, int64_t n, float lr, float b1, float b2,
-                                                  float eps, float c1, float c2)
-{
-    const int64_t i = blockIdx.x * static_cast<int64_t>(blockDim.x) + threadIdx.x;
-    if (i >= n) return;
-    const float gi = g[i];
-    const float mi = b1 * m[i] + (1.f - b1) * gi;
-    const float vi = b2 * v[i] + (1.f - b2) * gi * gi;
-    m[i] = mi;
-    v[i] = vi;
-    p[i] -= lr * (mi / c1) / (sqrtf(vi / c2) + eps);
-}
-
-// BF16 copies of a (rows x cols) FP32 weight: W row-major and W^T row-major.
-__global__ void __launch_bounds__(256) weightCopiesKernel(const float *__restrict__ w, int rows, int cols,
-                                                          __bf16 *__restrict__ wb, __bf16 *__restrict__ wtb)
-{
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= rows * cols) return;
-    const int r = i / cols, c = i % cols;
-    const __bf16 b = static_cast<__bf16>(w[i]);
-    wb[i] = b;
-    wtb[c * rows + r] = b;
-}
-
-// Rows of an FP32 (n x 24) feature table, standardised ((f - mean) / std), -> BF16 (rows x 32)
-// zero-padded, optional transpose; rows of the table are picked through `index` (a minibatch) or taken
-// in order when index is null. The matching targets are gathered into tOut (rows x 3) when given.
-__global__ void __launch_bounds__(256) packInputKernel(const float *__restrict__ f, const float *__restrict__ t,
-                                                       const int32_t *__restrict__ index,
-                                                       const float *__restrict__ mean, const float *__restrict__ invStd,
-                                                       int n, int rows, __bf16 *__restrict__ X, __bf16 *__restrict__ XT,
-                                                       float *__restrict__ tOut)
-{
-    const int64_t i = blockIdx.x * static_cast<int64_t>(blockDim.x) + threadIdx.x;
-    if (i >= static_cast<int64_t>(rows) * kMlpIn) return;
-    const int row = static_cast<int>(i / kMlpIn), col = static_cast<int>(i % kMlpIn);
-    float v = 0.f;
-    int src = -1;
-    if (row < n) src = index ? index[row] : row;
-    if (src >= 0 && col < kMlpFeatures) v = (f[static_cast<int64_t>(src) * kMlpFeatures + col] - mean[col]) * invStd[col];
-    const __bf16 b = static_cast<__bf16>(v);
-    X[i] = b;
-    if (XT) XT[static_cast<int64_t>(col) * rows + row] = b;
-    if (tOut && col < kMlpOut) tOut[static_cast<int64_t>(row) * kMlpOut + col] =
-        src >= 0 ? t[static_cast<int64_t>(src) * kMlpOut + col] : 0.f;
 }
 
 // ------------------------------------------------------------------------------------------------
@@ -202,34 +47,47 @@ constexpr int kNT = 4;  // 16-row tiles per wavefront task (each weight fragment
 constexpr int kTaskRows = 16 * kNT;
 constexpr int kBiasTotal = 3 * kMlpHidden + kMlpOutPad;
 
-__device__ __forceinline__ int permutedK(int kk, int q, int p) { return 32 * kk + (p < 4 ? 4 * q + p : 16 + 4 * q + p - 4); }
+// The backward pass multiplies by the transposed weights: A holds W^T (M = input features of the layer), K the layer's
+// outputs in the permuted order of the hidden layers (the last layer's 32 padded outputs in the plain order).
+constexpr int kFragT2 = kFragTotal, kFragT3 = kFragT2 + 2048, kFragT4 = kFragT3 + 2048, kFragAll = kFragT4 + 512;
 
-// frag[f][p] for every fragment of the fused kernel, from the padded FP32 master weights.
-__global__ void __launch_bounds__(256) mlpFragKernel(const float *__restrict__ w1, const float *__restrict__ w2,
-                                                     const float *__restrict__ w3, const float *__restrict__ w4,
-                                                     bf16x8 *__restrict__ frag)
+// Place of (row, k) of an operand in its fragments (in bf16 values): tiles of 16 rows, K steps of 32. In the permuted
+// order value p of lane quarter q holds k = 32 kk + (p < 4 ? 4 q + p : 16 + 4 q + p - 4), in the plain one 8 q + p.
+__device__ __forceinline__ int fragPlace(int row, int k, int ksteps, bool permuted)
 {
-    const int f = blockIdx.x * blockDim.x + threadIdx.x;
-    if (f >= kFragTotal) return;
-    const int lane = f & 63, q = lane >> 4, r16 = lane & 15;
-    const int t = f >> 6;  // (tile, kk) index within its layer
-    bf16x8 v;
-    if (f < kFragL2) {  // layer 1: 8 tiles x 1 step, plain K order, 32 padded inputs
-        const int i = t;
-#pragma unroll
-        for (int p = 0; p < 8; ++p) v[p] = static_cast<__bf16>(w1[(16 * i + r16) * kMlpIn + 8 * q + p]);
-    } else if (f < kFragL4) {  // layers 2, 3: 8 tiles x 4 steps
-        const float *w = f < kFragL3 ? w2 : w3;
-        const int tt = f < kFragL3 ? t - kFragL2 / 64 : t - kFragL3 / 64;
-        const int i = tt >> 2, kk = tt & 3;
-#pragma unroll
-        for (int p = 0; p < 8; ++p) v[p] = static_cast<__bf16>(w[(16 * i + r16) * kMlpHidden + permutedK(kk, q, p)]);
-    } else {  // layer 4: 1 tile (outputs 0..15 of the padded 32) x 4 steps
-        const int kk = t - kFragL4 / 64;
-#pragma unroll
-        for (int p = 0; p < 8; ++p) v[p] = static_cast<__bf16>(w4[r16 * kMlpHidden + permutedK(kk, q, p)]);
+    const int w = k & 31;
+    const int q = permuted ? (w & 15) >> 2 : w >> 3, p = permuted ? (w & 3) + (w & 16) / 4 : w & 7;
+    return (((row >> 4) * ksteps + (k >> 5)) * 64 + q * 16 + (row & 15)) * 8 + p;
+}
+
+// The padded master layout: per layer W (out x in, row-major), then its biases.
+constexpr int kW1 = 0, kB1 = kW1 + kMlpHidden * kMlpIn, kW2 = kB1 + kMlpHidden, kB2 = kW2 + kMlpHidden * kMlpHidden,
+              kW3 = kB2 + kMlpHidden, kB3 = kW3 + kMlpHidden * kMlpHidden, kW4 = kB3 + kMlpHidden,
+              kB4 = kW4 + kMlpOutPad * kMlpHidden;
+static_assert(kB4 + kMlpOutPad == kMlpPadded, "padded parameter count");
+
+// Writes parameter k of the padded layout, if it is a weight, to its places in the fragments.
+__device__ __forceinline__ void storeFrags(int k, float value, __bf16 *frag)
+{
+    const __bf16 v = static_cast<__bf16>(value);
+    if (k < kB1) {
+        frag[8 * kFragL1 + fragPlace(k / kMlpIn, k % kMlpIn, 1, false)] = v;
+    } else if ((k >= kW2 && k < kB2) || (k >= kW3 && k < kB3)) {
+        const bool second = k < kB2;
+        const int e = k - (second ? kW2 : kW3), o = e / kMlpHidden, i = e % kMlpHidden;
+        frag[8 * (second ? kFragL2 : kFragL3) + fragPlace(o, i, 4, true)] = v;
+        frag[8 * (second ? kFragT2 : kFragT3) + fragPlace(i, o, 4, true)] = v;
+    } else if (k >= kW4 && k < kB4) {
+        const int e = k - kW4, o = e / kMlpHidden, i = e % kMlpHidden;
+        if (o < 16) frag[8 * kFragL4 + fragPlace(o, i, 4, true)] = v;
+        frag[8 * kFragT4 + fragPlace(i, o, 1, false)] = v;
     }
-    frag[f] = v;
+}
+
+__global__ void __launch_bounds__(256) mlpFragKernel(const float *__restrict__ p, __bf16 *__restrict__ frag)
+{
+    const int k = blockIdx.x * blockDim.x + threadIdx.x;
+    if (k < kMlpPadded) storeFrags(k, p[k], frag);
 }
 
 __device__ __forceinline__ void hiddenEpilogue(const f32x4 (&acc)[8][kNT], const float *bias, int q,
@@ -344,67 +202,326 @@ __global__ void __launch_bounds__(256) mlpInferKernel(const float *__restrict__ 
     }
 }
 
+// ------------------------------------------------------------------------------------------------
+// The gradient of a batch: forward and backward of 64 rows per workgroup, 16 per wavefront, in one kernel.
+//
+// The layers run as in inference, rows as the B operand, activations and their gradients from layer to layer in
+// registers (SiLU' of the pre-activations stays there for the way back). A weight gradient sums over rows, dW = dZ^T H, so every
+// wavefront also stores its activations and dZ to LDS, features by rows, and the workgroup multiplies them with the 64
+// rows as K. Its sums over the row blocks it takes go to its own part of `partial`; mlpUpdateKernel adds the parts up in
+// a fixed order.
+//
+// What bounds it: latency. A minibatch of 4096 rows is 64 workgroups of about 400 MFMAs a wavefront; as separate
+// products (eleven of them, and 12 further launches) it took 420 us, most of it the weight gradients' serial K loop over
+// the batch in four workgroups. Now it is this kernel, 24 us, and mlpUpdateKernel, 7 us.
+constexpr int kTrainRows = 64;
+constexpr int kRowStride = kTrainRows + 8;  // bf16 per LDS feature row: 16-byte aligned, no bank conflicts
+constexpr int kSplit = 4;                   // threads that share a parameter's partial sums in mlpUpdateKernel
+
+// out[feature][row] of the tiles of v: this lane's features 16 i + 4 q + r of its row
+template <int TILES>
+__device__ __forceinline__ void storeRows(const f32x4 (&v)[TILES], __bf16 *out, int q, int row)
+{
+#pragma unroll
+    for (int i = 0; i < TILES; ++i)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) out[(16 * i + 4 * q + r) * kRowStride + row] = static_cast<__bf16>(v[i][r]);
+}
+
+// the tiles as B fragments of the next product (permuted K order)
+__device__ __forceinline__ void toFrags(const f32x4 (&v)[8], bf16x8 (&b)[4])
+{
+#pragma unroll
+    for (int kk = 0; kk < 4; ++kk)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            b[kk][r] = static_cast<__bf16>(v[2 * kk][r]);
+            b[kk][4 + r] = static_cast<__bf16>(v[2 * kk + 1][r]);
+        }
+}
+
+// The fragments as a buffer: a load is a scalar offset and the lane's, so the 148 loads of a row block need one address
+// register (as pointers each kept two of its own, and they spilled).
+typedef __attribute__((ext_vector_type(4))) uint32_t u32x4;
+__device__ __forceinline__ bf16x8 fragAt(__amdgpu_buffer_rsrc_t w, int f, int lane)
+{
+    return __builtin_bit_cast(bf16x8, static_cast<u32x4>(__builtin_amdgcn_raw_buffer_load_b128(w, lane * 16, f * 1024, 0)));
+}
+
+// acc = W b over 128 K: 8 tiles of 16 features, fragments in global memory, half of them loaded at once. The
+// compiler-level barrier keeps one product's loads from being issued with another's.
+__device__ __forceinline__ void product128(__amdgpu_buffer_rsrc_t w, int first, const bf16x8 (&b)[4], int lane, f32x4 (&acc)[8])
+{
+    asm volatile("" ::: "memory");
+#pragma unroll
+    for (int half = 0; half < 2; ++half) {
+        bf16x8 f[16];
+#pragma unroll
+        for (int k = 0; k < 16; ++k) f[k] = fragAt(w, first + 16 * half + k, lane);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            f32x4 &c = acc[4 * half + i];
+            c = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int kk = 0; kk < 4; ++kk) c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(f[4 * i + kk], b[kk], c, 0, 0, 0);
+        }
+    }
+}
+
+// v plus its value N lanes further round the 16 lanes of a row of the wavefront
+template <int N>
+__device__ __forceinline__ float addRotated(float v)
+{
+    return v + __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0x120 + N, 0xf, 0xf, true));
+}
+
+// Sums over the 16 rows of this wavefront (its lanes of one q), added to its own bias sums of the layer.
+template <int TILES>
+__device__ __forceinline__ void addBias(const f32x4 (&v)[TILES], float *sums, int q, int row16)
+{
+#pragma unroll
+    for (int i = 0; i < TILES; ++i) {
+        f32x4 t;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) t[r] = addRotated<8>(addRotated<4>(addRotated<2>(addRotated<1>(v[i][r]))));
+        if (row16 == 0) {
+            f32x4 *s = reinterpret_cast<f32x4 *>(sums + 16 * i + 4 * q);
+            *s += t;
+        }
+    }
+}
+
+// D H^T over the workgroup's rows, output features 16 tile0 .. and input features 16 ntile0 .., to (add: onto) out.
+template <int MT, int NT>
+__device__ __forceinline__ void weightGrad(const __bf16 *D, int tile0, const __bf16 *H, int ntile0, int q, int r16, int in,
+                                           float *out, bool add)
+{
+    f32x4 acc[MT][NT] = {};
+#pragma unroll
+    for (int ks = 0; ks < kTrainRows / 32; ++ks) {
+        bf16x8 d[MT];
+#pragma unroll
+        for (int m = 0; m < MT; ++m)
+            d[m] = *reinterpret_cast<const bf16x8 *>(D + (16 * (tile0 + m) + r16) * kRowStride + 32 * ks + 8 * q);
+#pragma unroll
+        for (int n = 0; n < NT; ++n) {
+            const bf16x8 h = *reinterpret_cast<const bf16x8 *>(H + (16 * (ntile0 + n) + r16) * kRowStride + 32 * ks + 8 * q);
+#pragma unroll
+            for (int m = 0; m < MT; ++m) acc[m][n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(d[m], h, acc[m][n], 0, 0, 0);
+        }
+    }
+#pragma unroll
+    for (int m = 0; m < MT; ++m)
+#pragma unroll
+        for (int n = 0; n < NT; ++n)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                float *o = out + (16 * (tile0 + m) + 4 * q + r) * in + 16 * (ntile0 + n) + r16;
+                *o = add ? *o + acc[m][n][r] : acc[m][n][r];
+            }
+}
+
+__global__ void __launch_bounds__(256, 1) mlpTrainKernel(MlpTrainArgs a)
+{
+    __shared__ __align__(16) __bf16 ht[3][kMlpHidden * kRowStride];
+    __shared__ __align__(16) __bf16 dt[3][kMlpHidden * kRowStride];
+    __shared__ __align__(16) __bf16 xt[kMlpIn * kRowStride];
+    __shared__ __align__(16) __bf16 yt[16 * kRowStride];
+    __shared__ __align__(16) float bias[4][3 * kMlpHidden + 16];
+    const int t = threadIdx.x, lane = t & 63, wave = t >> 6, q = lane >> 4, r16 = lane & 15;
+    for (int i = lane; i < 3 * kMlpHidden + 16; i += 64) bias[wave][i] = 0.f;  // a wavefront's own sums
+    // raw buffer of 32-bit elements
+    const __amdgpu_buffer_rsrc_t frag =
+        __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(a.frag), 0, kFragAll * sizeof(bf16x8), 0x00027000);
+    const float *b1 = a.params + kB1, *b2 = a.params + kB2, *b3 = a.params + kB3, *b4 = a.params + kB4;
+    float *out = a.partial + static_cast<int64_t>(blockIdx.x) * kMlpPadded;
+    double se = 0.0;
+    for (int block = blockIdx.x; block < a.rowBlocks; block += gridDim.x) {
+        // compiler-level memory barrier: the weight fragments are read again for every row block, not kept in registers
+        asm volatile("" ::: "memory");
+        const int lrow = wave * 16 + r16, row = block * kTrainRows + lrow;
+        const int src = row < a.n ? (a.index ? a.index[row] : row) : -1;
+        bf16x8 x = zeroFrag();
+        if (src >= 0 && q < 3) {
+            const float4 *f = reinterpret_cast<const float4 *>(a.features + static_cast<int64_t>(src) * kMlpFeatures + 8 * q);
+            const float4 u0 = f[0], u1 = f[1];
+            const float u[8] = {u0.x, u0.y, u0.z, u0.w, u1.x, u1.y, u1.z, u1.w};
+#pragma unroll
+            for (int p = 0; p < 8; ++p) x[p] = static_cast<__bf16>((u[p] - a.mean[8 * q + p]) * a.invStd[8 * q + p]);
+        }
+#pragma unroll
+        for (int p = 0; p < 8; ++p) xt[(8 * q + p) * kRowStride + lrow] = x[p];
+        // forward: z the pre-activations (then SiLU' of them, for the way back), h the activations
+        auto activate = [&](f32x4 (&z)[8], const float *b, __bf16 *out, bf16x8 (&next)[4]) {
+            f32x4 h[8];
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+                const f32x4 bi = *reinterpret_cast<const f32x4 *>(b + 16 * i + 4 * q);
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    const float v = z[i][r] + bi[r], sg = sigmoidf(v);
+                    h[i][r] = v * sg;
+                    z[i][r] = sg * (1.0f + v * (1.0f - sg));
+                }
+            }
+            storeRows(h, out, q, lrow);
+            toFrags(h, next);
+        };
+        f32x4 z1[8], z2[8], z3[8];
+        bf16x8 hb[4];
+#pragma unroll
+        for (int i = 0; i < 8; ++i)
+            z1[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fragAt(frag, kFragL1 / 64 + i, lane), x, f32x4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+        activate(z1, b1, ht[0], hb);
+        product128(frag, kFragL2 / 64, hb, lane, z2);
+        activate(z2, b2, ht[1], hb);
+        product128(frag, kFragL3 / 64, hb, lane, z3);
+        activate(z3, b3, ht[2], hb);
+        f32x4 y = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int kk = 0; kk < 4; ++kk)
+            y = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fragAt(frag, kFragL4 / 64 + kk, lane), hb[kk], y, 0, 0, 0);
+        // dY = 2 (y - t) / n on the real rows and outputs (features 0 .. 2: lanes of q 0), zero elsewhere
+        f32x4 dy[1] = {f32x4{0.f, 0.f, 0.f, 0.f}};
+        bf16x8 dyb = zeroFrag();
+        if (src >= 0 && q == 0) {
+            float e = 0.f;
+#pragma unroll
+            for (int r = 0; r < kMlpOut; ++r) {
+                const float d = y[r] + b4[r] - a.targets[static_cast<int64_t>(src) * kMlpOut + r];
+                e += d * d;
+                dy[0][r] = 2.0f * d / static_cast<float>(a.n);
+                dyb[r] = static_cast<__bf16>(dy[0][r]);
+            }
+            se += static_cast<double>(e);
+        }
+        storeRows(dy, yt, q, lrow);
+        addBias(dy, bias[wave] + 3 * kMlpHidden, q, r16);
+        // backward: dZ = (W^T dZ of the layer above) SiLU'
+        auto back = [&](f32x4 (&d)[8], const f32x4 (&z)[8], __bf16 *out, float *sums, bf16x8 (&next)[4]) {
+#pragma unroll
+            for (int i = 0; i < 8; ++i)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) d[i][r] *= z[i][r];
+            storeRows(d, out, q, lrow);
+            toFrags(d, next);
+            addBias(d, sums, q, r16);
+        };
+        f32x4 d[8];
+#pragma unroll
+        for (int i = 0; i < 8; ++i)
+            d[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fragAt(frag, kFragT4 / 64 + i, lane), dyb, f32x4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+        back(d, z3, dt[2], bias[wave] + 2 * kMlpHidden, hb);
+        product128(frag, kFragT3 / 64, hb, lane, d);
+        back(d, z2, dt[1], bias[wave] + kMlpHidden, hb);
+        product128(frag, kFragT2 / 64, hb, lane, d);
+        back(d, z1, dt[0], bias[wave], hb);
+        __syncthreads();
+        // wavefront w: output features 32 w .. of the hidden layers, input features 32 w .. of the last
+        const bool add = block != static_cast<int>(blockIdx.x);
+        weightGrad<1, 2>(yt, 0, ht[2], 2 * wave, q, r16, kMlpHidden, out + kW4, add);
+        weightGrad<2, 8>(dt[2], 2 * wave, ht[1], 0, q, r16, kMlpHidden, out + kW3, add);
+        weightGrad<2, 8>(dt[1], 2 * wave, ht[0], 0, q, r16, kMlpHidden, out + kW2, add);
+        weightGrad<2, 2>(dt[0], 2 * wave, xt, 0, q, r16, kMlpIn, out + kW1, add);
+        __syncthreads();
+    }
+    for (int i = t; i < 3 * kMlpHidden + 16; i += blockDim.x) {
+        const float v = ((bias[0][i] + bias[1][i]) + bias[2][i]) + bias[3][i];
+        const int layer = i / kMlpHidden, o = i % kMlpHidden;
+        out[(layer == 0 ? kB1 : layer == 1 ? kB2 : layer == 2 ? kB3 : kB4) + o] = v;
+    }
+    for (int o = 32; o > 0; o >>= 1) se += __shfl_down(se, o, 64);
+    __shared__ double waveSe[4];
+    if (lane == 0) waveSe[wave] = se;
+    __syncthreads();
+    if (t == 0) a.lossPartial[blockIdx.x] = ((waveSe[0] + waveSe[1]) + waveSe[2]) + waveSe[3];
+}
+
+// Whether parameter k of the padded layout has partial sums: outputs past the 16 that are computed have none.
+__device__ __forceinline__ bool trained(int k)
+{
+    return k < kW4 + 16 * kMlpHidden || (k >= kB4 && k < kB4 + 16);
+}
+
+// The gradient from the workgroups' partial sums (kSplit threads a parameter, each over a contiguous range of
+// workgroups, then in order), then, with ADAM (Kingma & Ba 2015), the new FP32 parameter and its places in the
+// operand fragments. The first workgroup also adds the batch's squared error to *loss.
+//
+// What bounds it: 10.6 MB of partial sums for 4096 rows, from the Infinity Cache.
+template <bool ADAM>
+__global__ void __launch_bounds__(256) mlpUpdateKernel(MlpUpdateArgs a)
+{
+    __shared__ float part[kSplit][64];
+    const int t = threadIdx.x & 63, seg = threadIdx.x >> 6, k = blockIdx.x * 64 + t;
+    float v = 0.f;
+    if (k < kMlpPadded && trained(k)) {
+        const int each = (a.parts + kSplit - 1) / kSplit, b = seg * each, e = min(b + each, a.parts);
+        const float *p = a.partial + static_cast<int64_t>(b) * kMlpPadded + k;
+        int i = b;
+        for (; i + 8 <= e; i += 8, p += 8 * kMlpPadded) {
+            float u[8];
+#pragma unroll
+            for (int j = 0; j < 8; ++j) u[j] = p[j * kMlpPadded];
+#pragma unroll
+            for (int j = 0; j < 8; ++j) v += u[j];
+        }
+        for (; i < e; ++i, p += kMlpPadded) v += *p;
+    }
+    part[seg][t] = v;
+    __syncthreads();
+    if (seg == 0 && k < kMlpPadded) {
+        float g = part[0][t];
+#pragma unroll
+        for (int j = 1; j < kSplit; ++j) g += part[j][t];
+        if constexpr (ADAM) {
+            const float mi = a.b1 * a.m[k] + (1.f - a.b1) * g;
+            const float vi = a.b2 * a.v[k] + (1.f - a.b2) * g * g;
+            a.m[k] = mi;
+            a.v[k] = vi;
+            const float w = a.params[k] - a.lr * (mi / a.c1) / (sqrtf(vi / a.c2) + a.eps);
+            a.params[k] = w;
+            storeFrags(k, w, static_cast<__bf16 *>(a.frag));
+        } else {
+            a.grad[k] = g;
+        }
+    }
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        double s = 0.0;
+        for (int i = 0; i < a.parts; ++i) s += a.lossPartial[i];
+        *a.loss += s;
+    }
+}
+
 inline int blocksFor(int64_t n, int bs) { return static_cast<int>((n + bs - 1) / bs); }
 
 }  // namespace
 
-hipError_t launchGemmNT(const __bf16 *A, int lda, const __bf16 *B, int ldb, int M, int N, int K, const GemmEpilogue &ep,
-                        hipStream_t stream)
+hipError_t launchMlpTrain(const MlpTrainArgs &a, int parts, hipStream_t stream)
 {
-    if (M % 16 || N % 16 || K % 32 || lda % 8 || ldb % 8 || M <= 0 || N <= 0 || K <= 0) return hipErrorInvalidValue;
-    dim3 grid((N + 63) / 64, (M + 63) / 64);
-    gemmNTKernel<<<grid, 256, 0, stream>>>(A, lda, B, ldb, M, N, K, ep);
+    if (a.n <= 0 || parts <= 0 || a.rowBlocks <= 0) return hipErrorInvalidValue;
+    mlpTrainKernel<<<parts, 256, 0, stream>>>(a);
     return hipGetLastError();
 }
 
-hipError_t launchLossGrad(const float *y, int ldy, const float *t, int outs, int n, int rows, int cols, float *dYf,
-                          __bf16 *dY, __bf16 *dYT, double *loss, hipStream_t stream)
+int mlpTrainBlocks(int64_t rows) { return static_cast<int>((rows + kTrainRows - 1) / kTrainRows); }
+
+hipError_t launchMlpUpdate(const MlpUpdateArgs &a, bool adam, hipStream_t stream)
 {
-    lossGradKernel<<<blocksFor(static_cast<int64_t>(rows) * cols, 256), 256, 0, stream>>>(y, ldy, t, outs, n, rows, cols,
-                                                                                       dYf, dY, dYT, loss);
+    const int grid = blocksFor(kMlpPadded, 64);
+    if (adam)
+        mlpUpdateKernel<true><<<grid, 256, 0, stream>>>(a);
+    else
+        mlpUpdateKernel<false><<<grid, 256, 0, stream>>>(a);
     return hipGetLastError();
 }
 
-hipError_t launchColSum(const float *m, int ld, int rows, int cols, float *out, hipStream_t stream)
+hipError_t launchMlpFrag(const float *params, void *frag, hipStream_t stream)
 {
-    colSumKernel<<<cols, 256, 0, stream>>>(m, ld, rows, out);
+    mlpFragKernel<<<blocksFor(kMlpPadded, 256), 256, 0, stream>>>(params, static_cast<__bf16 *>(frag));
     return hipGetLastError();
 }
 
-hipError_t launchAdam(float *p, const float *g, float *m, float *v, int64_t n, float lr, float b1, float b2, float eps,
-                      int64_t t, hipStream_t stream)
-{
-    const float c1 = 1.f - powf(b1, static_cast<float>(t)), c2 = 1.f - powf(b2, static_cast<float>(t));
-    adamKernel<<<blocksFor(n, 256), 256, 0, stream>>>(p, g, m, v, n, lr, b1, b2, eps, c1, c2);
-    return hipGetLastError();
-}
-
-hipError_t launchWeightCopies(const float *w, int rows, int cols, __bf16 *wb, __bf16 *wtb, hipStream_t stream)
-{
-    weightCopiesKernel<<<blocksFor(rows * cols, 256), 256, 0, stream>>>(w, rows, cols, wb, wtb);
-    return hipGetLastError();
-}
-
-hipError_t launchPackInput(const float *f, const float *t, const int32_t *index, const float *mean, const float *invStd,
-                           int n, int rows, __bf16 *X, __bf16 *XT, float *tOut, hipStream_t stream)
-{
-    packInputKernel<<<blocksFor(static_cast<int64_t>(rows) * kMlpIn, 256), 256, 0, stream>>>(f, t, index, mean, invStd,
-                                                                                           n, rows, X, XT, tOut);
-    return hipGetLastError();
-}
-
-}  // namespace spgvbd
-
-namespace spgvbd {
-
-hipError_t launchMlpFrag(const float *w1, const float *w2, const float *w3, const float *w4, void *frag,
-                         hipStream_t stream)
-{
-    mlpFragKernel<<<blocksFor(kFragTotal, 256), 256, 0, stream>>>(w1, w2, w3, w4, static_cast<bf16x8 *>(frag));
-    return hipGetLastError();
-}
-
-size_t mlpFragBytes() { return sizeof(bf16x8) * kFragTotal; }
+size_t mlpFragBytes() { return sizeof(bf16x8) * kFragAll; }
 
 hipError_t launchMlpInfer(const float *f, int n, const float *mean, const float *invStd, const void *frag,
                           const float *b1, const float *b2, const float *b3, const float *b4, float *y, int ldy,
