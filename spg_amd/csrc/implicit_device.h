@@ -74,7 +74,8 @@ hipError_t launchExpandSym(const SymBsr &A, double s, const int64_t *rowPtr, con
 struct CgScalars {
     double rhsNorm2, threshold, residualNorm2;
     double absNew[2];  // r.D^-1 r, by iteration parity
-    int32_t done;   // 1 once converged (or the right-hand side is 0)
+    int32_t done;   // 1 once converged (or the right-hand side is 0), 2 when the budget is spent
+    int32_t last;   // the iteration that found the solve over (-1 before the first, INT32_MAX: none yet)
     int32_t iters;  // completed iterations (Eigen's convention)
 };
 constexpr int kCgBlocks = 512;  // workgroups of the vector kernels (fixed: deterministic reductions)
@@ -82,11 +83,11 @@ constexpr int kCgBlocks = 512;  // workgroups of the vector kernels (fixed: dete
 // by launchCgInit) and uPartial of 2 kCgBlocks
 hipError_t launchCgInit(int64_t n, const double *b, const double *invdiag, double *x, double *r, double *p,
                         double *partial, CgScalars *s, double tol, hipStream_t stream);
-// iteration `iteration` (0-based, launch order): tmp = A p; alpha; x += alpha p, r -= alpha tmp;
+// iteration `iteration` (0-based, launch order): q = A p; alpha; x += alpha p, r -= alpha q;
 // convergence test; beta; p = D^-1 r + beta p. Three kernels. Non-null events are recorded right before and
 // after the product (to time it inside a solve).
 hipError_t launchCgIteration(const SymBsr &A, int64_t n, const double *invdiag, double *x, double *r, double *p,
-                             double *tmp, double *pPartial, double *uPartial, CgScalars *s, int32_t maxIters,
+                             double *q, double *pPartial, double *uPartial, CgScalars *s, int32_t maxIters,
                              int32_t iteration, hipStream_t stream, hipEvent_t spmvStart = nullptr,
                              hipEvent_t spmvEnd = nullptr);
 // invdiag = 1 / diagonal of A (1 where it is 0), from the diagonal blocks

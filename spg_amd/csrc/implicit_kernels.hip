@@ -186,50 +186,70 @@ __device__ __forceinline__ double blockSumFixed(double v, double *sh)
 constexpr int kSpmvG = 8;
 constexpr int kSpmvBlock = 1024;
 
+__device__ __forceinline__ V3<double> at3(const double *__restrict__ v, int64_t j)
+{
+    return {v[3 * j], v[3 * j + 1], v[3 * j + 2]};
+}
+// This lane's part of row `row` of A x
+__device__ __forceinline__ V3<double> symRowPart(const SymBsr &A, int64_t row, int lig, const double *__restrict__ x)
+{
+    V3<double> y = {0.0, 0.0, 0.0};
+    const int64_t u1 = A.upPtr[row + 1];
+    for (int64_t k = A.upPtr[row] + lig; k < u1; k += kSpmvG) {
+        const double *v = A.val + 9 * k;
+        const V3<double> xc = at3(x, A.upCol[k]);
+        y.x += v[0] * xc.x + v[1] * xc.y + v[2] * xc.z;
+        y.y += v[3] * xc.x + v[4] * xc.y + v[5] * xc.z;
+        y.z += v[6] * xc.x + v[7] * xc.y + v[8] * xc.z;
+    }
+    const int64_t l1 = A.loPtr[row + 1];
+    for (int64_t k = A.loPtr[row] + lig; k < l1; k += kSpmvG) {
+        const double *v = A.val + 9 * static_cast<int64_t>(A.loIdx[k]);
+        const V3<double> xc = at3(x, A.loCol[k]);
+        y.x += v[0] * xc.x + v[3] * xc.y + v[6] * xc.z;
+        y.y += v[1] * xc.x + v[4] * xc.y + v[7] * xc.z;
+        y.z += v[2] * xc.x + v[5] * xc.y + v[8] * xc.z;
+    }
+    return y;
+}
+
+__device__ __forceinline__ V3<double> rowSum(V3<double> y)
+{
+#pragma unroll
+    for (int o = kSpmvG / 2; o > 0; o >>= 1) {
+        y.x += __shfl_xor(y.x, o, kSpmvG);
+        y.y += __shfl_xor(y.y, o, kSpmvG);
+        y.z += __shfl_xor(y.z, o, kSpmvG);
+    }
+    return y;
+}
+
+__device__ __forceinline__ void store3(double *__restrict__ v, int64_t j, V3<double> a)
+{
+    v[3 * j] = a.x;
+    v[3 * j + 1] = a.y;
+    v[3 * j + 2] = a.z;
+}
+
+// cg: inside a solve, the product of iteration `iteration` (returns at once when the solve is over).
 __global__ void __launch_bounds__(kSpmvBlock) symSpmvKernel(SymBsr A, const double *__restrict__ x, double s,
                                                            double *__restrict__ y, double *__restrict__ partial,
-                                                           const int32_t *__restrict__ done)
+                                                           const CgScalars *__restrict__ cg, int32_t iteration)
 {
     __shared__ double sh[kSpmvBlock / 64];
-    if (done && *done) return;  // no other kernel runs meanwhile: the same value in every thread
+    if (cg && cg->last < iteration) return;
     const int32_t blk = xcdContiguous(static_cast<int32_t>(blockIdx.x), static_cast<int32_t>(gridDim.x));
     const int64_t t = blk * static_cast<int64_t>(kSpmvBlock) + threadIdx.x;
     const int64_t row = t / kSpmvG;
     const int lig = static_cast<int>(t % kSpmvG);
-    double y0 = 0.0, y1 = 0.0, y2 = 0.0;
-    if (row < A.rows) {
-        const int64_t u1 = A.upPtr[row + 1];
-        for (int64_t k = A.upPtr[row] + lig; k < u1; k += kSpmvG) {
-            const double *v = A.val + 9 * k;
-            const int64_t c = 3 * static_cast<int64_t>(A.upCol[k]);
-            const double x0 = x[c], x1 = x[c + 1], x2 = x[c + 2];
-            y0 += v[0] * x0 + v[1] * x1 + v[2] * x2;
-            y1 += v[3] * x0 + v[4] * x1 + v[5] * x2;
-            y2 += v[6] * x0 + v[7] * x1 + v[8] * x2;
-        }
-        const int64_t l1 = A.loPtr[row + 1];
-        for (int64_t k = A.loPtr[row] + lig; k < l1; k += kSpmvG) {
-            const double *v = A.val + 9 * static_cast<int64_t>(A.loIdx[k]);
-            const int64_t c = 3 * static_cast<int64_t>(A.loCol[k]);
-            const double x0 = x[c], x1 = x[c + 1], x2 = x[c + 2];
-            y0 += v[0] * x0 + v[3] * x1 + v[6] * x2;
-            y1 += v[1] * x0 + v[4] * x1 + v[7] * x2;
-            y2 += v[2] * x0 + v[5] * x1 + v[8] * x2;
-        }
-    }
-#pragma unroll
-    for (int o = kSpmvG / 2; o > 0; o >>= 1) {
-        y0 += __shfl_xor(y0, o, kSpmvG);
-        y1 += __shfl_xor(y1, o, kSpmvG);
-        y2 += __shfl_xor(y2, o, kSpmvG);
-    }
+    V3<double> r = {0.0, 0.0, 0.0};
+    if (row < A.rows) r = symRowPart(A, row, lig, x);
+    r = rowSum(r);
     double dot = 0.0;
     if (row < A.rows && lig == 0) {
-        const double z0 = s * y0, z1 = s * y1, z2 = s * y2;
-        y[3 * row] = z0;
-        y[3 * row + 1] = z1;
-        y[3 * row + 2] = z2;
-        dot = x[3 * row] * z0 + x[3 * row + 1] * z1 + x[3 * row + 2] * z2;
+        const V3<double> z = {s * r.x, s * r.y, s * r.z}, xr = at3(x, row);
+        store3(y, row, z);
+        dot = xr.x * z.x + xr.y * z.y + xr.z * z.z;
     }
     if (partial) {  // per-workgroup partial sums, in row order
         const double b = blockSumFixed(dot, sh);
@@ -321,102 +341,210 @@ __global__ void __launch_bounds__(1024) cgInitFinalKernel(const double *__restri
         const double th = tol * tol * bb;
         s->threshold = th > DBL_MIN ? th : DBL_MIN;
         s->done = (bb == 0.0 || bb < s->threshold) ? 1 : 0;
+        s->last = s->done ? -1 : INT32_MAX;
     }
 }
 
-// The sum of partial[0, n) in a fixed order, the same value in every thread (and every workgroup).
-__device__ __forceinline__ double blockTotal(const double *__restrict__ partial, int n, double *sh)
+// The sums of a[0, n) and b[0, n) (b may be null) in a fixed order, the same values in every thread and every
+// workgroup. In two parts, so that other work can go between the loads and the sum: thread t's entries t, t + B, t + 2B,
+// ... in that order, eight of its loads issued together; then one barrier. WAVES: wavefronts of the workgroup (B = 64
+// WAVES); sh: 2 WAVES values.
+template <int WAVES>
+__device__ __forceinline__ void threadTotals(const double *__restrict__ a, const double *__restrict__ b, int n, double &u,
+                                             double &v)
 {
-    // thread t adds entries t, t + B, t + 2B, ... in that order; eight of its loads are issued together
-    double acc = 0.0;
-    const int B = static_cast<int>(blockDim.x);
+    constexpr int B = 64 * WAVES;
+    u = v = 0.0;
     int i = threadIdx.x;
     for (; i + 7 * B < n; i += 8 * B) {
-        double v[8];
+        double x[8], y[8];
 #pragma unroll
-        for (int k = 0; k < 8; ++k) v[k] = partial[i + k * B];
+        for (int k = 0; k < 8; ++k) {
+            x[k] = a[i + k * B];
+            y[k] = b ? b[i + k * B] : 0.0;
+        }
 #pragma unroll
-        for (int k = 0; k < 8; ++k) acc += v[k];
+        for (int k = 0; k < 8; ++k) {
+            u += x[k];
+            v += y[k];
+        }
     }
-    for (; i < n; i += B) acc += partial[i];
-    const double t = blockSumFixed(acc, sh);
-    if (threadIdx.x == 0) sh[0] = t;
-    __syncthreads();
-    const double v = sh[0];
-    __syncthreads();
-    return v;
+    for (; i < n; i += B) {
+        u += a[i];
+        if (b) v += b[i];
+    }
 }
-
-// The flag read once per workgroup, so every thread of the workgroup takes the same branch.
-__device__ __forceinline__ bool blockDone(const CgScalars *s, int32_t *flag)
+template <int WAVES>
+__device__ __forceinline__ void blockTotals(double u, double v, double *sh, double &ta, double &tb)
 {
-    if (threadIdx.x == 0) *flag = s->done;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    for (int o = 32; o > 0; o >>= 1) {
+        u += __shfl_xor(u, o, 64);
+        v += __shfl_xor(v, o, 64);
+    }
+    if (lane == 0) {
+        sh[wave] = u;
+        sh[WAVES + wave] = v;
+    }
     __syncthreads();
-    return *flag != 0;
+    ta = tb = 0.0;
+#pragma unroll
+    for (int w = 0; w < WAVES; ++w) {
+        ta += sh[w];
+        tb += sh[WAVES + w];
+    }
 }
 
-// alpha = absNew / p.Ap (every workgroup reduces the product's partial sums itself, in the same order);
-// x += alpha p, r -= alpha A p; per-workgroup partial sums of r.r and r.D^-1 r.
+// Per-workgroup sums of u and v into a and b, fixed order.
+template <int WAVES>
+__device__ __forceinline__ void storeBlockSums(double u, double v, double *sh, double *a, double *b)
+{
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    for (int o = 32; o > 0; o >>= 1) {
+        u += __shfl_xor(u, o, 64);
+        v += __shfl_xor(v, o, 64);
+    }
+    __syncthreads();  // sh may still be read
+    if (lane == 0) {
+        sh[wave] = u;
+        sh[WAVES + wave] = v;
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        double s = 0.0, t = 0.0;
+        for (int w = 0; w < WAVES; ++w) {
+            s += sh[w];
+            t += sh[WAVES + w];
+        }
+        *a = s;
+        if (b) *b = t;
+    }
+}
+
+// The two vector kernels of an iteration. Workgroups take contiguous chunks of the vectors, renumbered so that each XCD's
+// chunks are the rows whose products it forms (symSpmvKernel): what one kernel writes the next finds in the same L2. Every
+// workgroup adds up the partial sums itself, in the same order; its first entries are loaded before that, since they do
+// not depend on the sum. A kernel of an iteration after `last` returns at once: the solve is over.
+//
+// What bounds them: on 200x200 cloths latency (launch, partial sums, entries, one after the other), on 512x512 cloths the
+// 44 and 25 MB they move. An iteration with its product took 21.9 us on a 48x48 cloth, 21.9 on 200x200, 36.9 on 330x330
+// and 61.8 on 512x512 where the sums were waited for before any entry was loaded and the chunks lay across the XCDs; it
+// takes 19.6, 19.3, 33.4 and 58.2. (One entry loaded ahead instead of four: about 65 us on 512x512. Both vector kernels folded
+// into the product, which then gathers two vectors: 19.2, 21, 38 and 70 us.)
+constexpr int kCgAhead = 4;  // entries of a thread loaded together
+
+// alpha = r.z / p.q, x += alpha p, r -= alpha q (q = A p); partial sums of r.r and r.D^-1 r.
 __global__ void __launch_bounds__(256) cgUpdateKernel(int64_t n, const double *__restrict__ invdiag,
                                                       double *__restrict__ x, double *__restrict__ r,
-                                                      const double *__restrict__ p, const double *__restrict__ tmp,
+                                                      const double *__restrict__ p, const double *__restrict__ q,
                                                       const double *__restrict__ pPartial, int nbP,
-                                                      double *__restrict__ partial, const CgScalars *s, int parity)
+                                                      double *__restrict__ partial, const CgScalars *s,
+                                                      int32_t iteration)
 {
-    __shared__ double sh[4];
-    __shared__ int32_t flag;
-    if (blockDone(s, &flag)) return;
-    const double alpha = s->absNew[parity] / blockTotal(pPartial, nbP, sh);
+    __shared__ double sh[8];
+    const int32_t last = s->last;
+    const double absNew = s->absNew[iteration & 1];
     const int64_t chunk = (n + gridDim.x - 1) / gridDim.x;
-    const int64_t b0 = blockIdx.x * chunk, e0 = b0 + chunk < n ? b0 + chunk : n;
+    const int64_t b0 = xcdContiguous(blockIdx.x, gridDim.x) * chunk, e0 = b0 + chunk < n ? b0 + chunk : n;
+    double xv[kCgAhead], pv[kCgAhead], rv[kCgAhead], qv[kCgAhead], dv[kCgAhead];
+    const auto load = [&](int64_t i0) {
+#pragma unroll
+        for (int k = 0; k < kCgAhead; ++k) {
+            const int64_t i = i0 + k * 256;
+            if (i < e0) {
+                xv[k] = x[i];
+                pv[k] = p[i];
+                rv[k] = r[i];
+                qv[k] = q[i];
+                dv[k] = invdiag[i];
+            }
+        }
+    };
+    int64_t i0 = b0 + threadIdx.x;
+    load(i0);
+    double u, v, pq, unused;
+    threadTotals<4>(pPartial, nullptr, nbP, u, v);
+    if (last < iteration) return;
+    blockTotals<4>(u, v, sh, pq, unused);
+    const double alpha = absNew / pq;
     double rr = 0.0, rz = 0.0;
-    for (int64_t i = b0 + threadIdx.x; i < e0; i += blockDim.x) {
-        x[i] += alpha * p[i];
-        const double ri = r[i] - alpha * tmp[i];
-        r[i] = ri;
-        rr += ri * ri;
-        rz += ri * (invdiag[i] * ri);
+    while (i0 < e0) {
+#pragma unroll
+        for (int k = 0; k < kCgAhead; ++k) {
+            const int64_t i = i0 + k * 256;
+            if (i < e0) {
+                const double ri = rv[k] - alpha * qv[k];
+                x[i] = xv[k] + alpha * pv[k];
+                r[i] = ri;
+                rr += ri * ri;
+                rz += ri * (dv[k] * ri);
+            }
+        }
+        i0 += kCgAhead * 256;
+        load(i0);
     }
-    const double a = blockSumFixed(rr, sh);
-    const double c = blockSumFixed(rz, sh);
-    if (threadIdx.x == 0) {
-        partial[blockIdx.x] = a;
-        partial[gridDim.x + blockIdx.x] = c;
-    }
+    storeBlockSums<4>(rr, rz, sh, partial + blockIdx.x, partial + gridDim.x + blockIdx.x);
 }
 
-// Convergence test and beta (every workgroup reduces the update's partial sums itself; workgroup 0
-// stores the scalars), then p = D^-1 r + beta p. absNew is double-buffered by iteration parity because
-// the other workgroups still read the old value while workgroup 0 stores the new one. A workgroup that
-// already sees the flag set by workgroup 0 skips p, which no later iteration reads.
+// The convergence test and beta = r.z / (r.z before); p = D^-1 r + beta p. Workgroup 0 stores the scalars while others
+// read them, so what they read is the same before and after: absNew is double-buffered by iteration parity, and `last`
+// stops later iterations only.
 __global__ void __launch_bounds__(256) cgDirectionKernel(int64_t n, const double *__restrict__ invdiag,
                                                          const double *__restrict__ r, double *__restrict__ p,
                                                          const double *__restrict__ uPartial, int nbU, CgScalars *s,
-                                                         int32_t maxIters, int parity)
+                                                         int32_t maxIters, int32_t iteration)
 {
-    __shared__ double sh[4];
-    __shared__ int32_t flag;
-    if (blockDone(s, &flag)) return;
-    const double rr = blockTotal(uPartial, nbU, sh);
-    const double rz = blockTotal(uPartial + nbU, nbU, sh);
+    __shared__ double sh[8];
+    const int32_t last = s->last;
+    const double before = s->absNew[iteration & 1], threshold = s->threshold;
+    const int64_t chunk = (n + gridDim.x - 1) / gridDim.x;
+    const int64_t b0 = xcdContiguous(blockIdx.x, gridDim.x) * chunk, e0 = b0 + chunk < n ? b0 + chunk : n;
+    double pv[kCgAhead], rv[kCgAhead], dv[kCgAhead];
+    const auto load = [&](int64_t i0) {
+#pragma unroll
+        for (int k = 0; k < kCgAhead; ++k) {
+            const int64_t i = i0 + k * 256;
+            if (i < e0) {
+                pv[k] = p[i];
+                rv[k] = r[i];
+                dv[k] = invdiag[i];
+            }
+        }
+    };
+    int64_t i0 = b0 + threadIdx.x;
+    load(i0);
+    double u, v, rr, rz;
+    threadTotals<4>(uPartial, uPartial + nbU, nbU, u, v);
+    if (last < iteration) return;
+    blockTotals<4>(u, v, sh, rr, rz);
     const bool lead = blockIdx.x == 0 && threadIdx.x == 0;
-    if (rr < s->threshold) {
+    if (rr < threshold) {
         if (lead) {
             s->residualNorm2 = rr;
+            s->last = iteration;
             s->done = 1;
         }
         return;
     }
-    const double beta = rz / s->absNew[parity];
+    const double beta = rz / before;
     if (lead) {
         s->residualNorm2 = rr;
-        s->absNew[parity ^ 1] = rz;
-        s->iters += 1;
-        if (s->iters >= maxIters) s->done = 2;  // iteration budget spent (x is the last iterate)
+        s->absNew[(iteration & 1) ^ 1] = rz;
+        s->iters = iteration + 1;
+        if (iteration + 1 >= maxIters) {  // iteration budget spent (x is the last iterate)
+            s->last = iteration;
+            s->done = 2;
+        }
     }
-    const int64_t chunk = (n + gridDim.x - 1) / gridDim.x;
-    const int64_t b0 = blockIdx.x * chunk, e0 = b0 + chunk < n ? b0 + chunk : n;
-    for (int64_t i = b0 + threadIdx.x; i < e0; i += blockDim.x) p[i] = invdiag[i] * r[i] + beta * p[i];
+    while (i0 < e0) {
+#pragma unroll
+        for (int k = 0; k < kCgAhead; ++k) {
+            const int64_t i = i0 + k * 256;
+            if (i < e0) p[i] = dv[k] * rv[k] + beta * pv[k];
+        }
+        i0 += kCgAhead * 256;
+        load(i0);
+    }
 }
 
 __global__ void __launch_bounds__(256) invDiagKernel(int64_t n, const int64_t *__restrict__ diagBlock,
@@ -547,7 +675,7 @@ int spmvPartials(int64_t rows) { return spmvGrid(rows); }
 hipError_t launchSymSpmv(const SymBsr &A, const double *x, double s, double *y, double *partial, hipStream_t stream)
 {
     if (A.rows <= 0) return hipSuccess;
-    symSpmvKernel<<<spmvGrid(A.rows), kSpmvBlock, 0, stream>>>(A, x, s, y, partial, nullptr);
+    symSpmvKernel<<<spmvGrid(A.rows), kSpmvBlock, 0, stream>>>(A, x, s, y, partial, nullptr, 0);
     return hipGetLastError();
 }
 
@@ -568,7 +696,7 @@ hipError_t launchCgInit(int64_t n, const double *b, const double *invdiag, doubl
 }
 
 hipError_t launchCgIteration(const SymBsr &A, int64_t n, const double *invdiag, double *x, double *r, double *p,
-                             double *tmp, double *pPartial, double *uPartial, CgScalars *s, int32_t maxIters,
+                             double *q, double *pPartial, double *uPartial, CgScalars *s, int32_t maxIters,
                              int32_t iteration, hipStream_t stream, hipEvent_t spmvStart, hipEvent_t spmvEnd)
 {
     if (spmvStart) {
@@ -576,14 +704,13 @@ hipError_t launchCgIteration(const SymBsr &A, int64_t n, const double *invdiag, 
         if (e != hipSuccess) return e;
     }
     const int grid = spmvGrid(A.rows);
-    symSpmvKernel<<<grid, kSpmvBlock, 0, stream>>>(A, p, 1.0, tmp, pPartial, &s->done);
+    symSpmvKernel<<<grid, kSpmvBlock, 0, stream>>>(A, p, 1.0, q, pPartial, s, iteration);
     if (spmvEnd) {
         const hipError_t e = hipEventRecord(spmvEnd, stream);
         if (e != hipSuccess) return e;
     }
-    const int parity = iteration & 1;
-    cgUpdateKernel<<<kCgBlocks, 256, 0, stream>>>(n, invdiag, x, r, p, tmp, pPartial, grid, uPartial, s, parity);
-    cgDirectionKernel<<<kCgBlocks, 256, 0, stream>>>(n, invdiag, r, p, uPartial, kCgBlocks, s, maxIters, parity);
+    cgUpdateKernel<<<kCgBlocks, 256, 0, stream>>>(n, invdiag, x, r, p, q, pPartial, grid, uPartial, s, iteration);
+    cgDirectionKernel<<<kCgBlocks, 256, 0, stream>>>(n, invdiag, r, p, uPartial, kCgBlocks, s, maxIters, iteration);
     return hipGetLastError();
 }
 
