@@ -50,24 +50,12 @@ RB_HD void matMulT3(const double *A, const double *B, double *C)
         for (int j = 0; j < 3; ++j)
             C[3 * i + j] = A[3 * i] * B[3 * j] + A[3 * i + 1] * B[3 * j + 1] + A[3 * i + 2] * B[3 * j + 2];
 }
-RB_HD void skew3(const double *v, double *S)
-{
-    S[0] = 0;
-    S[1] = -v[2];
-    S[2] = v[1];
-    S[3] = v[2];
-    S[4] = 0;
-    S[5] = -v[0];
-    S[6] = -v[1];
-    S[7] = v[0];
-    S[8] = 0;
-}
-
 // Rotation by `angle` about the unit axis a: Rodrigues' formula, rounded as Eigen's AngleAxis::toRotationMatrix
 // forms it (shared products (1 - c) a_i a_j for each symmetric pair).
 RB_HD void angleAxisToR(double angle, const double *a, double *R)
 {
-    const double c = cos(angle), sn = sin(angle);
+    double c, sn;
+    sincos(angle, &sn, &c);
     const double s0 = sn * a[0], s1 = sn * a[1], s2 = sn * a[2];
     const double c0 = (1 - c) * a[0], c1 = (1 - c) * a[1], c2 = (1 - c) * a[2];
     R[0] = c0 * a[0] + c;
@@ -156,8 +144,8 @@ RB_HD void addB(double *B, int i, int j, double v)
     }
 }
 
-// Adds J^T H_p J (J = [I, -[r]x]) into the 6x6 block B and J^T g into f with the given sign (the solve
-// accumulates forces, -gradient).
+// Adds J^T H_p J (J = [I, -[r]x], H_p symmetric) into the 6x6 block B and J^T g into f with the given sign (the solve
+// accumulates forces, -gradient). Products with [r]x are cross products with r: no term with a zero factor is formed.
 template <bool UPPER>
 RB_HD void addPointTerms(const double *r, const double *gp, const double *Hp, double gsign, double *f, double *B)
 {
@@ -168,25 +156,22 @@ RB_HD void addPointTerms(const double *r, const double *gp, const double *Hp, do
         f[d] -= gsign * gp[d];
         f[3 + d] -= gsign * rg[d];
     }
-    double S[9], HS[9], SH[9];
-    skew3(r, S);
-    // H (-S), S H, S H (-S)
+    double HS[9];  // -H [r]x, row by row; its transpose is [r]x H
 #pragma unroll
-    for (int i = 0; i < 3; ++i)
+    for (int i = 0; i < 3; ++i) cross3(r, Hp + 3 * i, HS + 3 * i);
 #pragma unroll
-        for (int j = 0; j < 3; ++j) {
-            HS[3 * i + j] = -(Hp[3 * i] * S[j] + Hp[3 * i + 1] * S[3 + j] + Hp[3 * i + 2] * S[6 + j]);
-            SH[3 * i + j] = S[3 * i] * Hp[j] + S[3 * i + 1] * Hp[3 + j] + S[3 * i + 2] * Hp[6 + j];
-        }
+    for (int j = 0; j < 3; ++j) {
+        const double col[3] = {HS[j], HS[3 + j], HS[6 + j]};
+        double rr[3];  // column j of -[r]x H [r]x
+        cross3(r, col, rr);
 #pragma unroll
-    for (int i = 0; i < 3; ++i)
-#pragma unroll
-        for (int j = 0; j < 3; ++j) {
+        for (int i = 0; i < 3; ++i) {
             addB<UPPER>(B, i, j, Hp[3 * i + j]);
             addB<UPPER>(B, i, 3 + j, HS[3 * i + j]);
-            addB<UPPER>(B, 3 + i, j, SH[3 * i + j]);
-            addB<UPPER>(B, 3 + i, 3 + j, -(SH[3 * i] * S[j] + SH[3 * i + 1] * S[3 + j] + SH[3 * i + 2] * S[6 + j]));
+            addB<UPPER>(B, 3 + j, i, HS[3 * i + j]);
+            addB<UPPER>(B, 3 + i, 3 + j, rr[i]);
         }
+    }
 }
 
 // One element's force (-gradient) and diagonal Hessian block for the body in `slot`, accumulated into f and B.
@@ -207,29 +192,26 @@ RB_HD void rbAccumulate(int type, int slot, const double *x0, const double *R0, 
     }
     if (type == kRbAlignment) {
         // C = sum_k |u_k x w_k|^2 with u_k, w_k the k-th columns of (I + [t0]x) R0 and (I + [t1]x) R1; E = 1/2 k C^2
-        // (rigidBodyOrientationAlignmentEnergy.cpp:15-31). With c_k = u_k x w_k: dc_k/dt0 = [w_k]x [u_k]x,
-        // dc_k/dt1 = -[u_k]x [w_k]x, and c_k is bilinear in (t0, t1), so d2C/dts2 = 2 sum_k J_k^T J_k.
+        // (rigidBodyOrientationAlignmentEnergy.cpp:15-31). With c_k = u_k x w_k and d_k = u_k . w_k:
+        // dc_k/dt0 = [w_k]x [u_k]x = u_k w_k^T - d_k I and dc_k/dt1 = -(w_k u_k^T - d_k I), J_k in either case; c_k is
+        // bilinear in (t0, t1) and orthogonal to both columns, so dC/dt0 = -2 sum_k d_k c_k = -dC/dt1 and
+        // d2C/dts2 = 2 sum_k J_k^T J_k, J_k^T J_k = |a|^2 b b^T - d_k (a b^T + b a^T) + d_k^2 I with a the slot's own
+        // column and b the other's.
+        const double *Ra = slot == 0 ? R0 : R1, *Rb = slot == 0 ? R1 : R0;
         double C = 0, g[3] = {0, 0, 0}, M[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
 #pragma unroll
         for (int k = 0; k < 3; ++k) {
-            const double u[3] = {R0[k], R0[3 + k], R0[6 + k]}, w[3] = {R1[k], R1[3 + k], R1[6 + k]};
-            double c[3], Su[9], Sw[9], J[9];
+            const double u[3] = {Ra[k], Ra[3 + k], Ra[6 + k]}, w[3] = {Rb[k], Rb[3 + k], Rb[6 + k]};
+            double c[3];
             cross3(u, w, c);
+            const double d = dot3(u, w), uu = dot3(u, u);
             C += dot3(c, c);
-            skew3(u, Su);
-            skew3(w, Sw);
-            if (slot == 0)
-                matMul3(Sw, Su, J);
-            else {
-                matMul3(Su, Sw, J);
-#pragma unroll
-                for (int q = 0; q < 9; ++q) J[q] = -J[q];
-            }
 #pragma unroll
             for (int i = 0; i < 3; ++i) {
-                g[i] += 2.0 * (J[i] * c[0] + J[3 + i] * c[1] + J[6 + i] * c[2]);
+                g[i] -= 2.0 * d * c[i];
 #pragma unroll
-                for (int j = 0; j < 3; ++j) M[3 * i + j] += J[i] * J[j] + J[3 + i] * J[3 + j] + J[6 + i] * J[6 + j];
+                for (int j = 0; j < 3; ++j)
+                    M[3 * i + j] += uu * (w[i] * w[j]) - d * (u[i] * w[j] + w[i] * u[j]) + (i == j ? d * d : 0.0);
             }
         }
         const double k = p[0];
@@ -285,17 +267,17 @@ RB_HD double solve6(double *H, const double *f, double *dx)
     for (int c = 0; c < 6; ++c) {
 #pragma unroll
         for (int r = c + 1; r < 6; ++r) {
-            const bool sw = fabs(H[6 * r + c]) > fabs(H[6 * c + c]);
+            if (!(fabs(H[6 * r + c]) > fabs(H[6 * c + c]))) continue;  // mostly so in every lane: then nothing is moved
 #pragma unroll
             for (int q = c; q < 6; ++q) {
-                const double hc = H[6 * c + q], hr = H[6 * r + q];
-                H[6 * c + q] = sw ? hr : hc;
-                H[6 * r + q] = sw ? hc : hr;
+                const double hc = H[6 * c + q];
+                H[6 * c + q] = H[6 * r + q];
+                H[6 * r + q] = hc;
             }
-            const double bc = b[c], br = b[r];
-            b[c] = sw ? br : bc;
-            b[r] = sw ? bc : br;
-            det = sw ? -det : det;
+            const double bc = b[c];
+            b[c] = b[r];
+            b[r] = bc;
+            det = -det;
         }
         const double d = H[6 * c + c];
         det *= d;

@@ -2,7 +2,7 @@
 // built from spg RigidBodyGroups, and the C-ABI.
 //
 // Layout in HBM. Bodies are renumbered colour-major ("slots"): the bodies of colour 0 of every group first, then
-// colour 1, ..., each colour a contiguous slot range that one launch covers (kRbLanes lanes per body). A slot's
+// colour 1, ..., each colour a contiguous slot range that one launch covers. A slot's
 // pose (centre and rotation matrix, 12 doubles = 96 bytes, read with 16-byte loads) is the record its neighbours
 // gather; the rest of its state is stored as arrays of 3 or 9 doubles per body (v, omega, theta, xt (inertial
 // prediction), xold, thetaold in 3; local inertia, its inverse and the rotation at the substep start in 9). World
@@ -33,10 +33,6 @@ using namespace spgrigid;
 namespace {
 
 constexpr int kRbBlock = 256;
-// Lanes cooperating on one body's incidence row in the colour solve. One lane per body measured fastest on a
-// 512 x 512 lattice (8 incidence entries per body): 78.7 us per sweep, against 82 with 2 lanes and 115 with 4; the
-// shuffle reduction stays for rows long enough to want more.
-constexpr int kRbLanes = 1;
 constexpr int kPose = 12;    // per-slot pose record: centre (3) then rotation matrix (9, row-major), 96 bytes
 
 struct RbState {
@@ -122,15 +118,13 @@ __global__ void __launch_bounds__(kRbBlock) rbBeginKernel(RbState s, int64_t nb,
         matMul3(dR, R, Rn);
         for (int k = 0; k < 9; ++k) R[k] = Rn[k];
     }
-    double thn[3], Rold[9];
-    rToAa(R, thn);
+    double Rold[9];
     aaToR(th, Rold);
     storePose(s.pose, b, x, R);
     for (int d = 0; d < 3; ++d) {
         s.xt[3 * b + d] = x[d];
         s.v[3 * b + d] = v[d];
         s.w[3 * b + d] = w[d];
-        s.th[3 * b + d] = thn[d];
     }
     for (int k = 0; k < 9; ++k) s.Rold[9 * b + k] = Rold[k];
 }
@@ -156,54 +150,47 @@ struct RbSolveArgs {
     double h;
 };
 
-// One colour: the 6x6 block descent of every body in [begin, end) (vbd.cpp:101-145 with the RigidBodyGroup
-// branches) and updateElementPositionFromDx (rigidBodyGroup.cpp:64-77). kRbLanes consecutive lanes share a body:
-// each sums every kRbLanes-th entry of its incidence row (lane 0 also the inertia terms) into a force and the
-// upper triangle of the block, the partial sums are combined by lane shuffles, and every lane of the group then
-// solves the same block; lane 0 writes the body.
-__global__ void __launch_bounds__(kRbBlock) rbSolveKernel(RbSolveArgs a, int64_t begin, int64_t end)
+// The terms of body b's inertia (mass, gyroscopic and rotational) in its force f and block Hu.
+__device__ __forceinline__ void inertiaTerms(const RbState &s, int64_t b, double invh, const double *x, const double *R,
+                                             double *f, double *Hu)
 {
-    const int32_t blk = xcdContiguousBlock(int32_t(blockIdx.x), int32_t(gridDim.x));
-    const int64_t t = int64_t(blk) * blockDim.x + threadIdx.x;
-    const int64_t b = begin + t / kRbLanes;
-    const int lane = int(t % kRbLanes);
-    if (b >= end) return;  // whole groups: kRbLanes divides the wavefront and the block
-    const RbState &s = a.s;
-    const double invh = 1.0 / a.h, invh2 = invh * invh;
-    double x[3], R[9], f[6], Hu[21];
+    const double invh2 = invh * invh;
+    const double mh2 = s.m[b] * invh2;
+    for (int d = 0; d < 3; ++d) f[d] = -mh2 * (x[d] - s.xt[3 * b + d]);
+    double wi[3], I[9], Il[9], Ro[9];
 #pragma unroll
-    for (int k = 0; k < 6; ++k) f[k] = 0.0;
-#pragma unroll
-    for (int k = 0; k < 21; ++k) Hu[k] = 0.0;
-    loadPose(s.pose, b, x, R);
-    if (lane == 0) {
-        const double mh2 = s.m[b] * invh2;
-        for (int d = 0; d < 3; ++d) f[d] = -mh2 * (x[d] - s.xt[3 * b + d]);
-        double wi[3], I[9], Il[9], Ro[9];
-#pragma unroll
-        for (int k = 0; k < 9; ++k) {
-            Il[k] = s.Il[9 * b + k];
-            Ro[k] = s.Rold[9 * b + k];
-        }
-        worldInertia(R, Il, I);
-        integratedOmega(R, Ro, invh, wi);
-        const double dw[3] = {wi[0] - s.w[3 * b], wi[1] - s.w[3 * b + 1], wi[2] - s.w[3 * b + 2]};
-        double Idw[3];
-        matVec3(I, dw, Idw);
-#pragma unroll
-        for (int d = 0; d < 3; ++d) {
-            f[3 + d] = -invh * Idw[d];
-            addB<true>(Hu, d, d, mh2);
-#pragma unroll
-            for (int q = 0; q < 3; ++q) addB<true>(Hu, 3 + d, 3 + q, invh2 * I[3 * d + q]);
-        }
+    for (int k = 0; k < 9; ++k) {
+        Il[k] = s.Il[9 * b + k];
+        Ro[k] = s.Rold[9 * b + k];
     }
-    const int64_t e0 = a.incPtr[b], e1 = a.incPtr[b + 1];
-    for (int64_t j = e0 + lane; j < e1; j += kRbLanes) {
-        const int2 en = a.inc[j];
-        const int type = kRbSpring + ((en.y >> 1) & 3);
-        const int slot = en.y & 1;
-        const double *pp = a.elemP + 2 * int64_t(uint32_t(en.y) >> 3);
+    worldInertia(R, Il, I);
+    integratedOmega(R, Ro, invh, wi);
+    const double dw[3] = {wi[0] - s.w[3 * b], wi[1] - s.w[3 * b + 1], wi[2] - s.w[3 * b + 2]};
+    double Idw[3];
+    matVec3(I, dw, Idw);
+#pragma unroll
+    for (int d = 0; d < 3; ++d) {
+        f[3 + d] = -invh * Idw[d];
+        addB<true>(Hu, d, d, mh2);
+#pragma unroll
+        for (int q = 0; q < 3; ++q) addB<true>(Hu, 3 + d, 3 + q, invh2 * I[3 * d + q]);
+    }
+}
+
+// Incidence entries first, first + step, ... of body b.
+__device__ __forceinline__ void incidenceTerms(const RbSolveArgs &a, int64_t b, int first, int step, const double *x,
+                                               const double *R, double *f, double *Hu)
+{
+    const int64_t e1 = a.incPtr[b + 1];
+    int64_t j = a.incPtr[b] + first;
+    int2 en = j < e1 ? a.inc[j] : make_int2(0, 0);
+    while (j < e1) {
+        const int other = en.x, desc = en.y;
+        j += step;
+        if (j < e1) en = a.inc[j];  // ahead of the terms: one link less in the chain of loads
+        const int type = kRbSpring + ((desc >> 1) & 3);
+        const int slot = desc & 1;
+        const double *pp = a.elemP + 2 * int64_t(uint32_t(desc) >> 3);
         double p[kRbParamStride];
         if (type == kRbAlignment) {
             p[0] = pp[0];
@@ -221,19 +208,67 @@ __global__ void __launch_bounds__(kRbBlock) rbSolveKernel(RbSolveArgs a, int64_t
             continue;
         }
         double xo[3], Ro[9];
-        loadPose(s.pose, en.x, xo, Ro);
+        loadPose(a.s.pose, other, xo, Ro);
         if (slot == 0)
             rbAccumulate<true>(type, 0, x, R, xo, Ro, p, f, Hu);
         else
             rbAccumulate<true>(type, 1, xo, Ro, x, R, p, f, Hu);
     }
+}
+
+// One colour: the 6x6 block descent of every body in [begin, end) (vbd.cpp:101-145 with the RigidBodyGroup
+// branches) and updateElementPositionFromDx (rigidBodyGroup.cpp:64-77; the rotation vectors follow in rbEndKernel).
+// A workgroup of WAVES wavefronts has 64 bodies, one to a lane. Wavefront 0 forms the inertia terms, the others share
+// the incidence row (with one wavefront it does both); their forces and upper triangles meet in LDS, and wavefront 0
+// adds them in order, solves and writes.
+//
+// What bounds it: the chain of dependent FP64 operations of one body (a logarithm of a rotation, its row, a 6x6 solve, a
+// rotation exponential), for the 220 registers leave two wavefronts on a SIMD and a colour of a 256x256 lattice has half a
+// wavefront for each. The row and the inertia are the parts that can go side by side. Lattices of n x n bodies (8 entries
+// a body), a step of ten sweeps over two colours in us, one body to a lane of one wavefront before and now with WAVES =
+// 1, 3, 4, 5, 6:
+//    32: 374   299  213  200  170  173        181: 351   287  217  208  187  191
+//   256: 388   329  292  268  332  337        362: 475   431  487  467  630  625        512: 760   682  790  811  1155  1179
+// Five wavefronts leave room for one workgroup on a compute unit, four for two; with more workgroups than that one
+// wavefront does it all, since then the chip is full of independent bodies. (Lanes of one wavefront sharing a body's row
+// have the inertia terms and the solve in their way: 230 us at 32, 397 at 256, four lanes to a body.)
+template <int WAVES>
+__global__ void __launch_bounds__(64 * WAVES) rbSolveKernel(RbSolveArgs a, int64_t begin, int64_t end)
+{
+    constexpr int kTerms = 27;
+    __shared__ double part[WAVES > 1 ? WAVES - 1 : 1][WAVES > 1 ? kTerms : 1][64];
+    const int32_t blk = xcdContiguousBlock(int32_t(blockIdx.x), int32_t(gridDim.x));
+    const int lane = int(threadIdx.x) & 63, wave = WAVES > 1 ? int(threadIdx.x) >> 6 : 0;
+    const int64_t b = begin + 64 * int64_t(blk) + lane;
+    const bool own = b < end;
+    double x[3], R[9], f[6], Hu[21];
 #pragma unroll
-    for (int m = 1; m < kRbLanes; m <<= 1) {
+    for (int k = 0; k < 6; ++k) f[k] = 0.0;
 #pragma unroll
-        for (int k = 0; k < 6; ++k) f[k] += __shfl_xor(f[k], m, kRbLanes);
-#pragma unroll
-        for (int k = 0; k < 21; ++k) Hu[k] += __shfl_xor(Hu[k], m, kRbLanes);
+    for (int k = 0; k < 21; ++k) Hu[k] = 0.0;
+    if (own) {
+        loadPose(a.s.pose, b, x, R);
+        if (wave == 0) inertiaTerms(a.s, b, 1.0 / a.h, x, R, f, Hu);
+        if (WAVES == 1 || wave > 0) incidenceTerms(a, b, WAVES > 1 ? wave - 1 : 0, WAVES > 1 ? WAVES - 1 : 1, x, R, f, Hu);
     }
+    if constexpr (WAVES > 1) {
+        if (wave > 0) {
+#pragma unroll
+            for (int k = 0; k < 6; ++k) part[wave - 1][k][lane] = f[k];
+#pragma unroll
+            for (int k = 0; k < 21; ++k) part[wave - 1][6 + k][lane] = Hu[k];
+        }
+        __syncthreads();
+        if (wave > 0) return;
+#pragma unroll
+        for (int w = 0; w < WAVES - 1; ++w) {
+#pragma unroll
+            for (int k = 0; k < 6; ++k) f[k] += part[w][k][lane];
+#pragma unroll
+            for (int k = 0; k < 21; ++k) Hu[k] += part[w][6 + k][lane];
+        }
+    }
+    if (!own) return;
     double H[36];
 #pragma unroll
     for (int i = 0; i < 6; ++i)
@@ -245,7 +280,6 @@ __global__ void __launch_bounds__(kRbBlock) rbSolveKernel(RbSolveArgs a, int64_t
         }
     double dx[6];
     const double det = solve6(H, f, dx);
-    if (lane != 0) return;
     if (det > 1e-10) {
         double xn[3];
         for (int d = 0; d < 3; ++d) xn[d] = x[d] + dx[d];
@@ -258,16 +292,14 @@ __global__ void __launch_bounds__(kRbBlock) rbSolveKernel(RbSolveArgs a, int64_t
 #pragma unroll
             for (int k = 0; k < 9; ++k) R[k] = Rn[k];
         }
-        double th[3];
-        rToAa(R, th);
-        storePose(s.pose, b, xn, R);
-        for (int d = 0; d < 3; ++d) s.th[3 * b + d] = th[d];
+        storePose(a.s.pose, b, xn, R);
     } else {
         atomicAdd(a.skipped, 1ull);
     }
 }
 
-// computeIntegratedVelocities (rigidBodyGroup.cpp:115-128)
+// computeIntegratedVelocities (rigidBodyGroup.cpp:115-128), and the rotation vectors of the final rotations: nothing reads
+// them between the substep's begin and here, so one launch forms them in place of every solve.
 __global__ void __launch_bounds__(kRbBlock) rbEndKernel(RbState s, int64_t nb, double invh)
 {
     const int64_t b = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
@@ -275,9 +307,13 @@ __global__ void __launch_bounds__(kRbBlock) rbEndKernel(RbState s, int64_t nb, d
     double x[3], R[9];
     loadPose(s.pose, b, x, R);
     for (int d = 0; d < 3; ++d) s.v[3 * b + d] = (x[d] - s.xold[3 * b + d]) * invh;
-    double w[3];
+    double w[3], th[3];
     integratedOmega(R, s.Rold + 9 * b, invh, w);
-    for (int d = 0; d < 3; ++d) s.w[3 * b + d] = w[d];
+    rToAa(R, th);
+    for (int d = 0; d < 3; ++d) {
+        s.w[3 * b + d] = w[d];
+        s.th[3 * b + d] = th[d];
+    }
 }
 
 __global__ void rbElementKernel(int type, int64_t n, const double *com, const double *rot, const double *prm,
@@ -303,7 +339,7 @@ thread_local std::string g_lastError;
 }  // namespace
 
 struct spg_rigid_ctx {
-    int device = 0;
+    int device = 0, cus = 1;
     hipStream_t stream = nullptr;
     std::string err;
     int64_t nb = 0, nElem = 0;
@@ -543,6 +579,13 @@ void buildContext(spg_rigid_ctx &c, const spg_rigid_group *groups, int32_t nGrou
     hipCheck(hipStreamSynchronize(c.stream), "hipStreamSynchronize");
 }
 
+// Wavefronts to a group of 64 bodies (figures at rbSolveKernel).
+int solveWaves(int64_t bodies, int cus)
+{
+    const int64_t groups = (bodies + 63) / 64;
+    return groups <= cus ? 5 : groups <= 2 * int64_t(cus) ? 4 : 1;
+}
+
 unsigned blocksFor(int64_t n) { return static_cast<unsigned>((n + kRbBlock - 1) / kRbBlock); }
 
 // One substep: begin, `iterations` sweeps over the colours, end. `events` (optional) brackets each colour launch.
@@ -561,7 +604,9 @@ void enqueueSubstep(spg_rigid_ctx &c, double h, int32_t iterations, const double
             const int64_t b0 = c.colorStart[col], b1 = c.colorStart[col + 1];
             if (b1 == b0) continue;
             if (events) hipCheck(hipEventRecord((*events)[ev].first, c.stream), "hipEventRecord");
-            hipLaunchKernelGGL(rbSolveKernel, dim3(blocksFor(kRbLanes * (b1 - b0))), dim3(kRbBlock), 0, c.stream, a, b0,
+            const int waves = solveWaves(b1 - b0, c.cus);
+            const auto kernel = waves == 5 ? rbSolveKernel<5> : waves == 4 ? rbSolveKernel<4> : rbSolveKernel<1>;
+            hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>((b1 - b0 + 63) / 64)), dim3(64 * waves), 0, c.stream, a, b0,
                                b1);
             hipCheck(hipGetLastError(), "solve launch");
             if (events) hipCheck(hipEventRecord((*events)[ev++].second, c.stream), "hipEventRecord");
@@ -592,6 +637,7 @@ int spg_rigid_create(spg_rigid_ctx **out, const spg_rigid_group *groups, int32_t
         if (device < 0 || device >= ndev) throw VbdError(SPG_VBD_ERR_INVALID, "invalid HIP device");
         c->device = device;
         hipCheck(hipSetDevice(device), "hipSetDevice");
+        hipCheck(hipDeviceGetAttribute(&c->cus, hipDeviceAttributeMultiprocessorCount, device), "hipDeviceGetAttribute");
         hipCheck(hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking), "hipStreamCreate");
         buildContext(*c, groups, n_groups);
     });
