@@ -57,7 +57,7 @@ struct spg_implicit_ctx {
     std::vector<int32_t> hCol;
     DevBuf<double> H, A, invdiag;  // upper blocks only
     // conjugate gradient
-    DevBuf<double> cgr, cgp, cgq, partial, partial2;
+    DevBuf<double> cgr, cgz, cgp, cgq, partial, partial2;
     DevBuf<CgScalars> cgs;
     CgScalars *hostCg = nullptr;  // pinned
     double *hostNorm = nullptr;   // pinned
@@ -127,7 +127,8 @@ struct spg_implicit_ctx {
         hipCheck(launchCombine(nUpper, H.p, c, np, upPtr.p, mass.p, a, A.p, stream), "combine launch");
         hipCheck(launchInvDiag(np, upPtr.p, A.p, invdiag.p, stream), "invdiag launch");
         timedBegin();
-        hipCheck(launchCgInit(ndof, b, invdiag.p, out, cgr.p, cgp.p, partial.p, cgs.p, tol, stream), "cg launch");
+        hipCheck(launchCgInit(ndof, b, invdiag.p, out, cgr.p, cgz.p, cgp.p, cgq.p, partial.p, cgs.p, tol, stream),
+                 "cg launch");
         // Iterations go in chunks; the scalars are read back after each chunk while the next one is
         // already queued, and every kernel of an iteration returns at once after convergence.
         constexpr int kChunk = 8;
@@ -149,7 +150,7 @@ struct spg_implicit_ctx {
                     e1 = spmvEvents[sampled.size()].second;
                     sampled.push_back(launched);
                 }
-                hipCheck(launchCgIteration(sym(A.p), ndof, invdiag.p, out, cgr.p, cgp.p, cgq.p,
+                hipCheck(launchCgIteration(sym(A.p), ndof, invdiag.p, out, cgr.p, cgz.p, cgp.p, cgq.p,
                                            partial.p, partial2.p, cgs.p, maxIters, launched, stream, e0, e1),
                          "cg launch");
             }
@@ -582,7 +583,7 @@ void buildContext(spg_implicit_ctx &c, const spg_vbd_object *objs, int32_t nObje
     c.H.alloc(9 * c.nUpper);
     c.A.alloc(9 * c.nUpper);
     c.invdiag.alloc(c.ndof);
-    for (auto *b : {&c.cgr, &c.cgp, &c.cgq, &c.x0, &c.v0, &c.vi, &c.dv, &c.rhs, &c.tmp, &c.xm1, &c.vm1})
+    for (auto *b : {&c.cgr, &c.cgz, &c.cgp, &c.cgq, &c.x0, &c.v0, &c.vi, &c.dv, &c.rhs, &c.tmp, &c.xm1, &c.vm1})
         b->alloc(c.ndof);
     c.partial.alloc(std::max<int64_t>(2 * kCgBlocks, spmvPartials(c.np)));
     c.partial2.alloc(2 * kCgBlocks);

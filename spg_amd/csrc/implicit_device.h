@@ -75,19 +75,20 @@ struct CgScalars {
     double rhsNorm2, threshold, residualNorm2;
     double absNew[2];  // r.D^-1 r, by iteration parity
     int32_t done;   // 1 once converged (or the right-hand side is 0), 2 when the budget is spent
-    int32_t last;   // the iteration that found the solve over (-1 before the first, INT32_MAX: none yet)
+    int32_t last;   // the iteration whose update ended the solve (-2: before the first; INT32_MAX: not yet)
     int32_t iters;  // completed iterations (Eigen's convention)
 };
 constexpr int kCgBlocks = 512;  // workgroups of the vector kernels (fixed: deterministic reductions)
 // a CG needs two partial-sum buffers: pPartial of max(2 kCgBlocks, spmvPartials(rows)) doubles (also used
 // by launchCgInit) and uPartial of 2 kCgBlocks
-hipError_t launchCgInit(int64_t n, const double *b, const double *invdiag, double *x, double *r, double *p,
-                        double *partial, CgScalars *s, double tol, hipStream_t stream);
-// iteration `iteration` (0-based, launch order): q = A p; alpha; x += alpha p, r -= alpha q;
-// convergence test; beta; p = D^-1 r + beta p. Three kernels. Non-null events are recorded right before and
-// after the product (to time it inside a solve).
-hipError_t launchCgIteration(const SymBsr &A, int64_t n, const double *invdiag, double *x, double *r, double *p,
-                             double *q, double *pPartial, double *uPartial, CgScalars *s, int32_t maxIters,
+hipError_t launchCgInit(int64_t n, const double *b, const double *invdiag, double *x, double *r, double *z, double *p,
+                        double *q, double *partial, CgScalars *s, double tol, hipStream_t stream);
+// iteration `iteration` (0-based, launch order) in two kernels: the convergence test and beta of the one before,
+// p = z + beta p, q = A z + beta q (= A p); alpha, x += alpha p, r -= alpha q, z = D^-1 r. The last one of the budget is
+// followed by its own test. Non-null events are recorded right before and after the first kernel (to time the product
+// inside a solve).
+hipError_t launchCgIteration(const SymBsr &A, int64_t n, const double *invdiag, double *x, double *r, double *z,
+                             double *p, double *q, double *pPartial, double *uPartial, CgScalars *s, int32_t maxIters,
                              int32_t iteration, hipStream_t stream, hipEvent_t spmvStart = nullptr,
                              hipEvent_t spmvEnd = nullptr);
 // invdiag = 1 / diagonal of A (1 where it is 0), from the diagonal blocks

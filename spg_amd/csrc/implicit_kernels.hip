@@ -3,6 +3,7 @@
 // do not depend on scheduling).
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cfloat>
 
 #include "implicit_device.h"
@@ -213,15 +214,42 @@ __device__ __forceinline__ V3<double> symRowPart(const SymBsr &A, int64_t row, i
     return y;
 }
 
+// v + the v of the lane that CTRL pairs this lane with: a permutation of the lanes of a row by the moving instruction
+// (DPP), without the hundred cycles of the LDS crossbar that a shuffle takes.
+template <int CTRL>
+__device__ __forceinline__ double addPartner(double v)
+{
+    const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(v), CTRL, 0xf, 0xf, true);
+    const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(v), CTRL, 0xf, 0xf, true);
+    return v + __hiloint2double(hi, lo);
+}
+// the sum over the 4, 8 or 16 lanes of each aligned group, in every lane of it: quads by exchange of neighbours and of
+// pairs, then mirrored halves and rows, whose quads hold equal sums by then
+template <int G>
+__device__ __forceinline__ double laneSum(double v)
+{
+    static_assert(G == 4 || G == 8 || G == 16, "lanes of a row");
+    v = addPartner<0xB1>(v);                         // quad_perm 1 0 3 2
+    v = addPartner<0x4E>(v);                         // quad_perm 2 3 0 1
+    if constexpr (G >= 8) v = addPartner<0x141>(v);  // row_half_mirror
+    if constexpr (G >= 16) v = addPartner<0x140>(v);  // row_mirror
+    return v;
+}
+__device__ __forceinline__ double lane(double v, int l)
+{
+    return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v), l), __builtin_amdgcn_readlane(__double2loint(v), l));
+}
+// the sum over the wavefront, in every lane (all of them active)
+__device__ __forceinline__ double waveSum(double v)
+{
+    v = laneSum<16>(v);
+    return (lane(v, 0) + lane(v, 16)) + (lane(v, 32) + lane(v, 48));
+}
+
 __device__ __forceinline__ V3<double> rowSum(V3<double> y)
 {
-#pragma unroll
-    for (int o = kSpmvG / 2; o > 0; o >>= 1) {
-        y.x += __shfl_xor(y.x, o, kSpmvG);
-        y.y += __shfl_xor(y.y, o, kSpmvG);
-        y.z += __shfl_xor(y.z, o, kSpmvG);
-    }
-    return y;
+    static_assert(kSpmvG == 8, "lanes of a block row");
+    return {laneSum<8>(y.x), laneSum<8>(y.y), laneSum<8>(y.z)};
 }
 
 __device__ __forceinline__ void store3(double *__restrict__ v, int64_t j, V3<double> a)
@@ -231,13 +259,10 @@ __device__ __forceinline__ void store3(double *__restrict__ v, int64_t j, V3<dou
     v[3 * j + 2] = a.z;
 }
 
-// cg: inside a solve, the product of iteration `iteration` (returns at once when the solve is over).
 __global__ void __launch_bounds__(kSpmvBlock) symSpmvKernel(SymBsr A, const double *__restrict__ x, double s,
-                                                           double *__restrict__ y, double *__restrict__ partial,
-                                                           const CgScalars *__restrict__ cg, int32_t iteration)
+                                                           double *__restrict__ y, double *__restrict__ partial)
 {
     __shared__ double sh[kSpmvBlock / 64];
-    if (cg && cg->last < iteration) return;
     const int32_t blk = xcdContiguous(static_cast<int32_t>(blockIdx.x), static_cast<int32_t>(gridDim.x));
     const int64_t t = blk * static_cast<int64_t>(kSpmvBlock) + threadIdx.x;
     const int64_t row = t / kSpmvG;
@@ -306,7 +331,8 @@ __device__ __forceinline__ double finalSum(const double *__restrict__ partial, i
 
 __global__ void __launch_bounds__(256) cgInitKernel(int64_t n, const double *__restrict__ b,
                                                     const double *__restrict__ invdiag, double *__restrict__ x,
-                                                    double *__restrict__ r, double *__restrict__ p,
+                                                    double *__restrict__ r, double *__restrict__ z,
+                                                    double *__restrict__ p, double *__restrict__ q,
                                                     double *__restrict__ partial)
 {
     __shared__ double sh[4];
@@ -316,7 +342,9 @@ __global__ void __launch_bounds__(256) cgInitKernel(int64_t n, const double *__r
         const double bi = b[i];
         x[i] = 0.0;
         r[i] = bi;
-        p[i] = invdiag[i] * bi;
+        z[i] = invdiag[i] * bi;
+        p[i] = 0.0;
+        q[i] = 0.0;
     }
     const double bb = chunkSum(n, [&](int64_t i) { return b[i] * b[i]; }, sh);
     const double rp = chunkSum(n, [&](int64_t i) { return b[i] * (invdiag[i] * b[i]); }, sh);
@@ -341,7 +369,7 @@ __global__ void __launch_bounds__(1024) cgInitFinalKernel(const double *__restri
         const double th = tol * tol * bb;
         s->threshold = th > DBL_MIN ? th : DBL_MIN;
         s->done = (bb == 0.0 || bb < s->threshold) ? 1 : 0;
-        s->last = s->done ? -1 : INT32_MAX;
+        s->last = s->done ? -2 : INT32_MAX;
     }
 }
 
@@ -374,25 +402,25 @@ __device__ __forceinline__ void threadTotals(const double *__restrict__ a, const
         if (b) v += b[i];
     }
 }
+// The totals of the wavefronts' sums in sh, in every lane.
+template <int WAVES>
+__device__ __forceinline__ void wavesTotal(const double *sh, int lane, double &ta, double &tb)
+{
+    ta = laneSum<WAVES>(sh[lane % WAVES]);
+    tb = laneSum<WAVES>(sh[WAVES + lane % WAVES]);
+}
 template <int WAVES>
 __device__ __forceinline__ void blockTotals(double u, double v, double *sh, double &ta, double &tb)
 {
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    for (int o = 32; o > 0; o >>= 1) {
-        u += __shfl_xor(u, o, 64);
-        v += __shfl_xor(v, o, 64);
-    }
+    u = waveSum(u);
+    v = waveSum(v);
     if (lane == 0) {
         sh[wave] = u;
         sh[WAVES + wave] = v;
     }
     __syncthreads();
-    ta = tb = 0.0;
-#pragma unroll
-    for (int w = 0; w < WAVES; ++w) {
-        ta += sh[w];
-        tb += sh[WAVES + w];
-    }
+    wavesTotal<WAVES>(sh, lane, ta, tb);
 }
 
 // Per-workgroup sums of u and v into a and b, fixed order.
@@ -400,43 +428,117 @@ template <int WAVES>
 __device__ __forceinline__ void storeBlockSums(double u, double v, double *sh, double *a, double *b)
 {
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    for (int o = 32; o > 0; o >>= 1) {
-        u += __shfl_xor(u, o, 64);
-        v += __shfl_xor(v, o, 64);
-    }
+    u = waveSum(u);
+    v = waveSum(v);
     __syncthreads();  // sh may still be read
     if (lane == 0) {
         sh[wave] = u;
         sh[WAVES + wave] = v;
     }
     __syncthreads();
-    if (threadIdx.x == 0) {
-        double s = 0.0, t = 0.0;
-        for (int w = 0; w < WAVES; ++w) {
-            s += sh[w];
-            t += sh[WAVES + w];
-        }
-        *a = s;
-        if (b) *b = t;
+    if (wave > 0) return;
+    wavesTotal<WAVES>(sh, lane, u, v);
+    if (lane == 0) {
+        *a = u;
+        if (b) *b = v;
     }
 }
 
-// The two vector kernels of an iteration. Workgroups take contiguous chunks of the vectors, renumbered so that each XCD's
-// chunks are the rows whose products it forms (symSpmvKernel): what one kernel writes the next finds in the same L2. Every
-// workgroup adds up the partial sums itself, in the same order; its first entries are loaded before that, since they do
-// not depend on the sum. A kernel of an iteration after `last` returns at once: the solve is over.
-//
-// What bounds them: on 200x200 cloths latency (launch, partial sums, entries, one after the other), on 512x512 cloths the
-// 44 and 25 MB they move. An iteration with its product took 21.9 us on a 48x48 cloth, 21.9 on 200x200, 36.9 on 330x330
-// and 61.8 on 512x512 where the sums were waited for before any entry was loaded and the chunks lay across the XCDs; it
-// takes 19.6, 19.3, 33.4 and 58.2. (One entry loaded ahead instead of four: about 65 us on 512x512. Both vector kernels folded
-// into the product, which then gathers two vectors: 19.2, 21, 38 and 70 us.)
-constexpr int kCgAhead = 4;  // entries of a thread loaded together
+// The end of CG iteration `iteration` - 1 from its sums rr = r.r and rz = r.D^-1 r: the convergence test, and beta. False:
+// the solve is over. The first thread of the first workgroup (`lead`) stores the scalars while other workgroups read
+// them, so what they read is the same before and after: absNew is double-buffered by iteration parity, and `last` is
+// compared so that it ends later kernels only.
+__device__ __forceinline__ bool cgNext(CgScalars *s, double rr, double rz, double before, double threshold,
+                                       int32_t iteration, bool lead, double &beta)
+{
+    beta = rz / before;
+    if (lead) s->residualNorm2 = rr;
+    if (rr < threshold) {
+        if (lead) {
+            s->last = iteration - 1;
+            s->done = 1;
+        }
+        return false;
+    }
+    if (lead) {
+        s->absNew[iteration & 1] = rz;
+        s->iters = iteration;
+    }
+    return true;
+}
 
-// alpha = r.z / p.q, x += alpha p, r -= alpha q (q = A p); partial sums of r.r and r.D^-1 r.
+// An iteration in two kernels. The first closes the iteration before (convergence, beta) and forms p = z + beta p and
+// q = A p = A z + beta q, z = D^-1 r: the product is taken of z, which the kernel before left whole, so no kernel in
+// between has to form p for the gather, and its loads do not wait for beta. The second (cgUpdateKernel) takes alpha and
+// updates x, r and z. Every workgroup adds up the partial sums itself, in the same order, and loads its first entries
+// before that.
+//
+// What bounds an iteration: at 200x200 particles the latency of two dependent launches with a reduction each (the matrix,
+// 20 MB, comes from the L2s; the product takes 10.1 us of the 15.8, 8.1 by itself), at 512x512 the 0.13 GB of the matrix.
+// In three kernels (product, update, direction p = z + beta p), whose sums waited for each other through shuffles, an
+// iteration took 22.4 us at 48x48 particles, 18.7 at 100x100, 21.9 at 200x200, 37.0 at 330x330 and 61.4 at 512x512; now
+// 14.4, 11.5, 15.8, 31.2 and 59.3. Of that the sums by lane permutations are 2 to 3 us, workgroups of 512 instead of 1024
+// threads 1.5 (the barrier waits for fewer). Forming p in the gather (z + beta p of every neighbour) took 19.2, 15.7, 21,
+// 38 and 70. The recurrence for q costs no accuracy: after 1517 iterations at 200x200 particles b - A x is 9.7347e-11 |b|
+// and the r that was carried along 9.7350e-11 |b| (9.7229e-11 and 9.7228e-11 with q = A p).
+constexpr int kCgProductBlock = 512;
+__global__ void __launch_bounds__(kCgProductBlock) cgProductKernel(SymBsr A, const double *__restrict__ z,
+                                                              double *__restrict__ p, double *__restrict__ q,
+                                                              const double *__restrict__ uPartial,
+                                                              double *__restrict__ partial, CgScalars *s,
+                                                              int32_t iteration)
+{
+    constexpr int WAVES = kCgProductBlock / 64;
+    __shared__ double sh[2 * WAVES];
+    const int32_t last = s->last;
+    const double before = s->absNew[(iteration & 1) ^ 1], threshold = s->threshold;
+    const int32_t blk = xcdContiguous(static_cast<int32_t>(blockIdx.x), static_cast<int32_t>(gridDim.x));
+    const int64_t t = blk * static_cast<int64_t>(kCgProductBlock) + threadIdx.x;
+    const int64_t row = t / kSpmvG;
+    const int lig = static_cast<int>(t % kSpmvG);
+    const bool store = row < A.rows && lig == 0;
+    double u = 0.0, v = 0.0;
+    static_assert(kCgBlocks <= kCgProductBlock, "a partial sum to a thread");
+    if (iteration > 0 && threadIdx.x < kCgBlocks) {
+        u = uPartial[threadIdx.x];
+        v = uPartial[kCgBlocks + threadIdx.x];
+    }
+    // `last` is iteration - 1 at the most while this kernel may store it (cgNext): every thread takes the same branch
+    if (last < iteration - 1) return;
+    V3<double> zr = {0.0, 0.0, 0.0}, pr = zr, qr = zr, w = zr;
+    if (row < A.rows) w = symRowPart(A, row, lig, z);
+    __builtin_amdgcn_sched_barrier(0);  // the row's own entries after its product's: together they exceed 64 registers
+    if (store) {
+        zr = at3(z, row);
+        pr = at3(p, row);
+        qr = at3(q, row);
+    }
+    w = rowSum(w);
+    double beta = 0.0;
+    if (iteration > 0) {
+        double rr, rz;
+        blockTotals<WAVES>(u, v, sh, rr, rz);
+        if (!cgNext(s, rr, rz, before, threshold, iteration, blockIdx.x == 0 && threadIdx.x == 0, beta)) return;
+    }
+    double dot = 0.0;
+    if (store) {
+        pr = {zr.x + beta * pr.x, zr.y + beta * pr.y, zr.z + beta * pr.z};
+        qr = {w.x + beta * qr.x, w.y + beta * qr.y, w.z + beta * qr.z};
+        store3(p, row, pr);
+        store3(q, row, qr);
+        dot = pr.x * qr.x + pr.y * qr.y + pr.z * qr.z;
+    }
+    storeBlockSums<WAVES>(dot, 0.0, sh, partial + blk, nullptr);
+}
+
+// alpha = r.z / p.q, x += alpha p, r -= alpha q, z = D^-1 r; partial sums of r.r and r.z. Workgroups take contiguous
+// chunks of the vectors, renumbered so that each XCD's chunks are the rows whose products it forms: what one kernel
+// writes the next finds in the same L2.
+constexpr int kCgAhead = 4;  // entries of a thread loaded together
 __global__ void __launch_bounds__(256) cgUpdateKernel(int64_t n, const double *__restrict__ invdiag,
                                                       double *__restrict__ x, double *__restrict__ r,
-                                                      const double *__restrict__ p, const double *__restrict__ q,
+                                                      double *__restrict__ z, const double *__restrict__ p,
+                                                      const double *__restrict__ q,
                                                       const double *__restrict__ pPartial, int nbP,
                                                       double *__restrict__ partial, const CgScalars *s,
                                                       int32_t iteration)
@@ -473,11 +575,12 @@ __global__ void __launch_bounds__(256) cgUpdateKernel(int64_t n, const double *_
         for (int k = 0; k < kCgAhead; ++k) {
             const int64_t i = i0 + k * 256;
             if (i < e0) {
-                const double ri = rv[k] - alpha * qv[k];
+                const double ri = rv[k] - alpha * qv[k], zi = dv[k] * ri;
                 x[i] = xv[k] + alpha * pv[k];
                 r[i] = ri;
+                z[i] = zi;
                 rr += ri * ri;
-                rz += ri * (dv[k] * ri);
+                rz += ri * zi;
             }
         }
         i0 += kCgAhead * 256;
@@ -486,64 +589,20 @@ __global__ void __launch_bounds__(256) cgUpdateKernel(int64_t n, const double *_
     storeBlockSums<4>(rr, rz, sh, partial + blockIdx.x, partial + gridDim.x + blockIdx.x);
 }
 
-// The convergence test and beta = r.z / (r.z before); p = D^-1 r + beta p. Workgroup 0 stores the scalars while others
-// read them, so what they read is the same before and after: absNew is double-buffered by iteration parity, and `last`
-// stops later iterations only.
-__global__ void __launch_bounds__(256) cgDirectionKernel(int64_t n, const double *__restrict__ invdiag,
-                                                         const double *__restrict__ r, double *__restrict__ p,
-                                                         const double *__restrict__ uPartial, int nbU, CgScalars *s,
-                                                         int32_t maxIters, int32_t iteration)
+// After the last iteration of the budget: its convergence test (x is the last iterate either way).
+__global__ void __launch_bounds__(256) cgFinishKernel(const double *__restrict__ uPartial, int nbU, CgScalars *s,
+                                                      int32_t iterations)
 {
     __shared__ double sh[8];
+    double u, v, rr, rz, beta;
     const int32_t last = s->last;
-    const double before = s->absNew[iteration & 1], threshold = s->threshold;
-    const int64_t chunk = (n + gridDim.x - 1) / gridDim.x;
-    const int64_t b0 = xcdContiguous(blockIdx.x, gridDim.x) * chunk, e0 = b0 + chunk < n ? b0 + chunk : n;
-    double pv[kCgAhead], rv[kCgAhead], dv[kCgAhead];
-    const auto load = [&](int64_t i0) {
-#pragma unroll
-        for (int k = 0; k < kCgAhead; ++k) {
-            const int64_t i = i0 + k * 256;
-            if (i < e0) {
-                pv[k] = p[i];
-                rv[k] = r[i];
-                dv[k] = invdiag[i];
-            }
-        }
-    };
-    int64_t i0 = b0 + threadIdx.x;
-    load(i0);
-    double u, v, rr, rz;
+    const double before = s->absNew[(iterations & 1) ^ 1], threshold = s->threshold;
     threadTotals<4>(uPartial, uPartial + nbU, nbU, u, v);
-    if (last < iteration) return;
+    if (last < iterations) return;
     blockTotals<4>(u, v, sh, rr, rz);
-    const bool lead = blockIdx.x == 0 && threadIdx.x == 0;
-    if (rr < threshold) {
-        if (lead) {
-            s->residualNorm2 = rr;
-            s->last = iteration;
-            s->done = 1;
-        }
-        return;
-    }
-    const double beta = rz / before;
-    if (lead) {
-        s->residualNorm2 = rr;
-        s->absNew[(iteration & 1) ^ 1] = rz;
-        s->iters = iteration + 1;
-        if (iteration + 1 >= maxIters) {  // iteration budget spent (x is the last iterate)
-            s->last = iteration;
-            s->done = 2;
-        }
-    }
-    while (i0 < e0) {
-#pragma unroll
-        for (int k = 0; k < kCgAhead; ++k) {
-            const int64_t i = i0 + k * 256;
-            if (i < e0) p[i] = dv[k] * rv[k] + beta * pv[k];
-        }
-        i0 += kCgAhead * 256;
-        load(i0);
+    if (cgNext(s, rr, rz, before, threshold, iterations, threadIdx.x == 0, beta) && threadIdx.x == 0) {
+        s->last = iterations - 1;
+        s->done = 2;
     }
 }
 
@@ -670,12 +729,13 @@ namespace {
 int spmvGrid(int64_t rows) { return blocksFor(rows * kSpmvG, kSpmvBlock); }
 }  // namespace
 
-int spmvPartials(int64_t rows) { return spmvGrid(rows); }
+int cgProductGrid(int64_t rows) { return blocksFor(rows * kSpmvG, kCgProductBlock); }
+int spmvPartials(int64_t rows) { return std::max(spmvGrid(rows), cgProductGrid(rows)); }
 
 hipError_t launchSymSpmv(const SymBsr &A, const double *x, double s, double *y, double *partial, hipStream_t stream)
 {
     if (A.rows <= 0) return hipSuccess;
-    symSpmvKernel<<<spmvGrid(A.rows), kSpmvBlock, 0, stream>>>(A, x, s, y, partial, nullptr, 0);
+    symSpmvKernel<<<spmvGrid(A.rows), kSpmvBlock, 0, stream>>>(A, x, s, y, partial);
     return hipGetLastError();
 }
 
@@ -687,30 +747,30 @@ hipError_t launchExpandSym(const SymBsr &A, double s, const int64_t *rowPtr, con
     return hipGetLastError();
 }
 
-hipError_t launchCgInit(int64_t n, const double *b, const double *invdiag, double *x, double *r, double *p,
-                        double *partial, CgScalars *s, double tol, hipStream_t stream)
+hipError_t launchCgInit(int64_t n, const double *b, const double *invdiag, double *x, double *r, double *z, double *p,
+                        double *q, double *partial, CgScalars *s, double tol, hipStream_t stream)
 {
-    cgInitKernel<<<kCgBlocks, 256, 0, stream>>>(n, b, invdiag, x, r, p, partial);
+    cgInitKernel<<<kCgBlocks, 256, 0, stream>>>(n, b, invdiag, x, r, z, p, q, partial);
     cgInitFinalKernel<<<1, 1024, 0, stream>>>(partial, kCgBlocks, s, tol);
     return hipGetLastError();
 }
 
-hipError_t launchCgIteration(const SymBsr &A, int64_t n, const double *invdiag, double *x, double *r, double *p,
-                             double *q, double *pPartial, double *uPartial, CgScalars *s, int32_t maxIters,
+hipError_t launchCgIteration(const SymBsr &A, int64_t n, const double *invdiag, double *x, double *r, double *z,
+                             double *p, double *q, double *pPartial, double *uPartial, CgScalars *s, int32_t maxIters,
                              int32_t iteration, hipStream_t stream, hipEvent_t spmvStart, hipEvent_t spmvEnd)
 {
     if (spmvStart) {
         const hipError_t e = hipEventRecord(spmvStart, stream);
         if (e != hipSuccess) return e;
     }
-    const int grid = spmvGrid(A.rows);
-    symSpmvKernel<<<grid, kSpmvBlock, 0, stream>>>(A, p, 1.0, q, pPartial, s, iteration);
+    const int grid = cgProductGrid(A.rows);
+    cgProductKernel<<<grid, kCgProductBlock, 0, stream>>>(A, z, p, q, uPartial, pPartial, s, iteration);
     if (spmvEnd) {
         const hipError_t e = hipEventRecord(spmvEnd, stream);
         if (e != hipSuccess) return e;
     }
-    cgUpdateKernel<<<kCgBlocks, 256, 0, stream>>>(n, invdiag, x, r, p, q, pPartial, grid, uPartial, s, iteration);
-    cgDirectionKernel<<<kCgBlocks, 256, 0, stream>>>(n, invdiag, r, p, uPartial, kCgBlocks, s, maxIters, iteration);
+    cgUpdateKernel<<<kCgBlocks, 256, 0, stream>>>(n, invdiag, x, r, z, p, q, pPartial, grid, uPartial, s, iteration);
+    if (iteration + 1 == maxIters) cgFinishKernel<<<1, 256, 0, stream>>>(uPartial, kCgBlocks, s, maxIters);
     return hipGetLastError();
 }
 
