@@ -6,8 +6,8 @@
 #include <cmath>
 #include <limits>
 #include <numeric>
-#include <system_error>
-#include <thread>
+
+#include "host_threads.h"
 
 namespace spgvbd {
 
@@ -22,24 +22,6 @@ constexpr int kPlanThreads = 8;         // host threads that build the plan
 
 // a round of one group in a tile
 double groupUs(int32_t type) { return type == 4 ? 1.6 : type <= 5 ? 1.0 : 2.5; }
-
-// Runs f(0) .. f(n - 1) on the host threads.
-template <class F>
-void forAll(int64_t n, F &&f)
-{
-    std::atomic<int64_t> next{0};
-    auto work = [&] {
-        for (int64_t k; (k = next.fetch_add(1)) < n;) f(k);
-    };
-    std::vector<std::thread> threads;
-    threads.reserve(kPlanThreads);
-    try {
-        while (static_cast<int64_t>(threads.size()) + 1 < std::min<int64_t>(kPlanThreads, n)) threads.emplace_back(work);
-    } catch (const std::system_error &) {  // no further thread to be had
-    }
-    work();
-    for (auto &t : threads) t.join();
-}
 
 // Bisects particles [b, e) of `order` along the longer side of their box, again and again, into `parts` ranges of equal
 // size; writes the ranges' ends to ends[0 .. parts).
@@ -67,7 +49,7 @@ void bisect(const float *xyz, int stride, int32_t *order, int64_t b, int64_t e, 
         return u != v ? u < v : p < q;
     });
     if (e - b > 65536) {
-        forAll(2, [&](int64_t k) {
+        forAll(2, kPlanThreads, [&](int64_t k) {
             if (k == 0)
                 bisect(xyz, stride, order, b, mid, left, ends);
             else
@@ -131,7 +113,7 @@ class Holders {
   public:
     Holders(int64_t nv, const std::vector<TileGroup> &groups) : m_nv(nv), m_of(nv * groups.size())
     {
-        forAll(groups.size(), [&](int64_t g) {
+        forAll(groups.size(), kPlanThreads, [&](int64_t g) {
             int32_t *of = m_of.data() + g * nv;
             std::fill(of, of + nv, -1);
             for (int32_t s = 0; s < groups[g].count; ++s)
@@ -277,7 +259,7 @@ bool fill(TilePlan &plan, const Tiles &tiles, const Holders &holders, const std:
         std::vector<Built> built(nt);
         std::atomic<bool> ok{true};
         const int64_t chunk = std::max<int64_t>(1, nt / (8 * kPlanThreads));
-        forAll((nt + chunk - 1) / chunk, [&](int64_t c) {
+        forAll((nt + chunk - 1) / chunk, kPlanThreads, [&](int64_t c) {
             Grower grower(holders, groups);
             std::vector<std::vector<int32_t>> stencils(batch.groups);
             for (int64_t t = c * chunk; t < std::min(nt, (c + 1) * chunk) && ok; ++t) {
@@ -330,7 +312,7 @@ bool fill(TilePlan &plan, const Tiles &tiles, const Holders &holders, const std:
         }
         plan.particles.resize(particleAt[nt]);
         plan.entries.resize(entryAt[nt]);
-        forAll(nt, [&](int64_t t) {
+        forAll(nt, kPlanThreads, [&](int64_t t) {
             std::copy(built[t].particles.begin(), built[t].particles.end(), plan.particles.begin() + particleAt[t]);
             std::copy(built[t].entries.begin(), built[t].entries.end(), plan.entries.begin() + entryAt[t]);
         });
@@ -349,7 +331,7 @@ TilePlan buildTilePlan(const float *xyz, int stride, const std::vector<int64_t> 
     if (nv == 0 || groups.size() < 2) return {};
     if (nv * static_cast<int64_t>(groups.size()) > kHoldersMax) return {};
     std::vector<std::vector<int32_t>> stencilsOf(groups.size());
-    forAll(groups.size(), [&](int64_t g) {
+    forAll(groups.size(), kPlanThreads, [&](int64_t g) {
         stencilsOf[g].resize(static_cast<size_t>(groups[g].count) * groups[g].size);
         stencils(static_cast<int32_t>(g), stencilsOf[g].data());
         groups[g].stencils = stencilsOf[g].data();
@@ -359,7 +341,7 @@ TilePlan buildTilePlan(const float *xyz, int stride, const std::vector<int64_t> 
     for (double margin : {1.125, 1.5, 2.0}) {
         std::array<std::vector<TileBatch>, 3> batches;
         std::array<double, 3> us;
-        forAll(3, [&](int64_t k) {
+        forAll(3, kPlanThreads, [&](int64_t k) {
             if (k > 0 && tiles[k].count() == tiles[k - 1].count()) {  // small objects: the same tiles
                 us[k] = std::numeric_limits<double>::max();
                 return;
