@@ -7,11 +7,9 @@
 // with pageable copies of all records, 1.21 ms now; of 24 objects advanced together (each of whose reads copied all 24):
 // 9.2 ms, 1.26 ms now; of a 256x256 rigid-body lattice 1.43 ms, 0.68 ms now.
 #include <algorithm>
-#include <atomic>
 #include <cstring>
-#include <system_error>
-#include <thread>
 
+#include "host_threads.h"
 #include "state_io.h"
 
 namespace spgvbd {
@@ -118,29 +116,11 @@ void StateReader::read(const Field3<T> *fields, int count, const int32_t *order,
             hipCheck(hipEventRecord(m_events[k], stream), "hipEventRecord");
         }
         hipCheck(hipEventSynchronize(m_events[0]), "hipEventSynchronize");
-        std::atomic<int64_t> next{0};
-        std::atomic<int> failed{hipSuccess};
-        auto work = [&] {
-            for (int64_t k; (k = next.fetch_add(1)) < now;) {
-                const hipError_t e = hipEventSynchronize(m_events[k]);
-                if (e != hipSuccess) {
-                    failed = e;
-                    return;
-                }
-                const int64_t first = (p0 + k) * part, m = std::min(part, n - first);
-                for (int f = 0; f < nf; ++f)
-                    widen(host + k * partValues + f * 3 * m, use[f].dst + 3 * first, 3 * m);
-            }
-        };
-        std::vector<std::thread> threads;
-        try {
-            threads.reserve(kThreads);
-            while (static_cast<int64_t>(threads.size()) + 1 < std::min<int64_t>(kThreads, now)) threads.emplace_back(work);
-        } catch (const std::system_error &) {  // no further thread to be had: those that started do it
-        }
-        work();
-        for (auto &t : threads) t.join();
-        hipCheck(static_cast<hipError_t>(failed.load()), "hipEventSynchronize");
+        forAll(now, kThreads, [&](int64_t k) {
+            hipCheck(hipEventSynchronize(m_events[k]), "hipEventSynchronize");
+            const int64_t first = (p0 + k) * part, m = std::min(part, n - first);
+            for (int f = 0; f < nf; ++f) widen(host + k * partValues + f * 3 * m, use[f].dst + 3 * first, 3 * m);
+        });
     }
 }
 
