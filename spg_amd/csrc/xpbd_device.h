@@ -77,7 +77,7 @@ hipError_t launchXpbdBegin(float4 *pos, float4 *vel, float4 *xold, int32_t n, fl
                            hipStream_t stream);
 hipError_t launchXpbdBoundary(float4 *pos, float4 *xold, int32_t n, float invhPrev, float h, float gx, float gy,
                               float gz, hipStream_t stream);
-// copy: where not null, x is written there too.
+// copy: where not null, x is written there too (it may be xold).
 hipError_t launchXpbdEnd(const float4 *pos, const float4 *xold, float4 *vel, int32_t n, float invh,
                          hipStream_t stream, float4 *copy = nullptr);
 

@@ -421,9 +421,10 @@ __global__ void __launch_bounds__(256) xpbdBoundaryKernel(float4 *__restrict__ p
     pos[i] = x;
 }
 
-__global__ void __launch_bounds__(256) xpbdEndKernel(const float4 *__restrict__ pos, const float4 *__restrict__ xold,
-                                                     float4 *__restrict__ vel, int32_t n, float invh,
-                                                     float4 *__restrict__ copy)
+// `copy` (where not null) may be xold itself, the start of a step of one substep: each thread reads its entry before it
+// writes it, so neither is __restrict__.
+__global__ void __launch_bounds__(256) xpbdEndKernel(const float4 *pos, const float4 *xold, float4 *__restrict__ vel,
+                                                     int32_t n, float invh, float4 *copy)
 {
     const int32_t i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;

@@ -71,3 +71,18 @@ def test_tiles_bitwise_equal_single_launches(name, parallel):
         assert fa == fb, (name, nsub)
     if name == "stiff cube":
         assert fa > 0
+
+
+@pytest.mark.parametrize("nsub", [1, 2, 3, 4, 5, 6, 7])
+def test_substep_counts(nsub):
+    """The position buffers change roles every substep: with one batch to a substep, a step of 1, 4, 7 ... substeps ends
+    with its start in the buffer that receives the new positions, whose velocities need it."""
+    ctx = {}
+    for runs in (0, 1):
+        ctx[runs] = native.XpbdContext([_cloth(24).xpbd_object()])
+        ctx[runs].set_launch(group_runs=runs)
+        for _ in range(2):
+            ctx[runs].step(scenes.DT, nsub, scenes.GRAVITY)
+    (x0, v0), (x1, v1) = ctx[0].state(), ctx[1].state()
+    assert np.array_equal(x0, x1) and np.array_equal(v0, v1)
+    assert np.abs(v1).max() > 0.1  # gravity over two frames: 0.33 m/s where the cloth falls freely
