@@ -3,6 +3,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <new>
 #include <stdexcept>
 #include <string>
 #include <vector>
@@ -19,6 +20,26 @@ struct VbdError : std::runtime_error {
 inline void hipCheck(hipError_t e, const char *what)
 {
     if (e != hipSuccess) throw VbdError(SPG_VBD_ERR_HIP, std::string(what) + ": " + hipGetErrorString(e));
+}
+
+// The device has no memory for an allocation.
+struct DeviceMemoryError : VbdError {
+    using VbdError::VbdError;
+};
+
+// Runs f, which allocates memory that can be done without. False where the host or the device has none for it; any other
+// error passes through.
+template <class F>
+bool ifMemoryAllows(F &&f)
+{
+    try {
+        f();
+        return true;
+    } catch (const std::bad_alloc &) {
+    } catch (const DeviceMemoryError &) {
+        (void)hipGetLastError();  // or the next launch would be blamed for it
+    }
+    return false;
 }
 
 template <class T>
@@ -39,7 +60,11 @@ struct DevBuf {
     {
         release();
         if (count == 0) return;
-        hipCheck(hipMalloc(reinterpret_cast<void **>(&p), count * sizeof(T)), "hipMalloc");
+        const hipError_t e = hipMalloc(reinterpret_cast<void **>(&p), count * sizeof(T));
+        if (e != hipSuccess) p = nullptr;
+        if (e == hipErrorOutOfMemory)
+            throw DeviceMemoryError(SPG_VBD_ERR_HIP, std::string("hipMalloc: ") + hipGetErrorString(e));
+        hipCheck(e, "hipMalloc");
         n = count;
     }
     // grows to at least `count` elements (contents are not kept)

@@ -447,12 +447,13 @@ void validateEnergy(const spg_xpbd_energy &e, int64_t np)
 void buildTiles(spg_xpbd_ctx &c, const std::vector<float4> &x, const std::vector<TileGroup> &groups,
                 const std::function<void(int32_t, int32_t *)> &stencils)
 {
-    try {
+    TilePlan plan;
+    DevBuf<TileEntry> entries;
+    DevBuf<int64_t> segmentEntry;
+    const bool fits = ifMemoryAllows([&] {
         for (const auto &g : groups) c.tilesSet = std::max(c.tilesSet, tileSet(g.type));
-        const TilePlan plan = buildTilePlan(x.empty() ? nullptr : &x[0].x, 4, c.objOffset, groups, stencils, tileThreads(c.tilesSet));
+        plan = buildTilePlan(x.empty() ? nullptr : &x[0].x, 4, c.objOffset, groups, stencils, tileThreads(c.tilesSet));
         if (plan.batches.empty()) return;
-        DevBuf<TileEntry> entries;
-        DevBuf<int64_t> segmentEntry;
         c.tileHeaders.upload(plan.headers, c.stream);
         c.tileParticles.upload(plan.particles, c.stream);
         c.tileSegments.upload(plan.segments, c.stream);
@@ -463,19 +464,17 @@ void buildTiles(spg_xpbd_ctx &c, const std::vector<float4> &x, const std::vector
         hipCheck(launchTileRecords(c.args(0.f), c.tileSegments.p, static_cast<int32_t>(plan.segments.size()),
                                    segmentEntry.p, entries.p, c.tileRecords.p, c.stream),
                  "tile records launch");
-        hipCheck(hipStreamSynchronize(c.stream), "hipStreamSynchronize");
-        c.batches = plan.batches;
-    } catch (const std::bad_alloc &) {
-    } catch (const VbdError &) {
-        (void)hipGetLastError();
+    });
+    hipCheck(hipStreamSynchronize(c.stream), "hipStreamSynchronize");  // the lists end here
+    if (fits) {
+        c.batches = std::move(plan.batches);
+        return;
     }
-    if (c.batches.empty()) {
-        c.tileHeaders.release();
-        c.tileParticles.release();
-        c.tileSegments.release();
-        c.tileRecords.release();
-        c.spare.release();
-    }
+    c.tileHeaders.release();
+    c.tileParticles.release();
+    c.tileSegments.release();
+    c.tileRecords.release();
+    c.spare.release();
 }
 
 void buildContext(spg_xpbd_ctx &c, const spg_xpbd_object *objs, int32_t nObjects)
