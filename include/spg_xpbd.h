@@ -79,7 +79,8 @@ typedef struct {
 } spg_xpbd_object;
 
 typedef struct {
-    int32_t block_size; /* threads per workgroup of the projection kernels: 64, 128 or 256 */
+    int32_t block_size; /* threads per workgroup of the projection kernels that run one stencil group: 64, 128 or 256
+                           (a launch over tiles has its own size) */
     int32_t use_graph;  /* 1: capture a whole step in a hipGraph and replay it */
     int32_t group_runs; /* 1 (default): consecutive stencil groups run in one launch where that is faster: over
                            tiles of particles, each with the part of its neighbours it depends on; in timed steps
@@ -103,6 +104,16 @@ typedef struct {
     double type_bytes[14];
 } spg_xpbd_stats;
 
+/* A substep as an untimed step launches it, with the launch shape's group runs. */
+typedef struct {
+    int32_t launches;       /* projection launches */
+    int32_t tiled_launches; /* of them over tiles of particles; 0: none, each group (or run of small groups) by itself */
+    int64_t tiles;          /* workgroups of the tiled launches */
+    int64_t tile_particles; /* particles they load, each other's among them */
+    int64_t tile_projections; /* stencils they project: those two tiles depend on are projected by both */
+    int64_t tile_bytes;     /* device memory of the tiles' records and lists, kept by the context */
+} spg_xpbd_substep_plan;
+
 typedef struct spg_xpbd_ctx spg_xpbd_ctx;
 
 /* parallel_gauss_seidel: 1 = XPBD(true) (stencil colour groups), 0 = XPBD(false) (serial order). */
@@ -119,6 +130,8 @@ int spg_xpbd_get_groups(const spg_xpbd_ctx *ctx, int32_t object, int32_t energy,
 /* Projection kernel launches per substep of a timed step (all objects together), with the launch shape's group
    runs. */
 int spg_xpbd_num_launches(const spg_xpbd_ctx *ctx, int32_t *n);
+/* The launches of an untimed step's substep. */
+int spg_xpbd_get_substep_plan(const spg_xpbd_ctx *ctx, spg_xpbd_substep_plan *plan);
 
 int spg_xpbd_set_state(spg_xpbd_ctx *ctx, int32_t object, const double *x, const double *v);
 int spg_xpbd_get_state(spg_xpbd_ctx *ctx, int32_t object, double *x, double *v);

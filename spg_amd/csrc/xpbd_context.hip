@@ -128,6 +128,7 @@ struct spg_xpbd_ctx {
     DevBuf<int32_t> tileParticles;
     DevBuf<TileSegment> tileSegments;
     DevBuf<float4> tileRecords, spare;  // spare: third position buffer
+    int64_t tileProjections = 0;        // stencils projected by the tiles of a substep
 
     spg_xpbd_launch launch{256, 1, 1};
     bool timing = false;
@@ -284,9 +285,11 @@ struct spg_xpbd_ctx {
                  "end launch");
     }
 
+    bool tiled() const { return launch.group_runs && !batches.empty(); }
+
     void enqueueStep(double dt, int32_t nsub, const double *g, bool timed)
     {
-        if (launch.group_runs && !timed && !batches.empty()) {
+        if (tiled() && !timed) {
             enqueueTiledStep(dt, nsub, g);
             return;
         }
@@ -468,6 +471,7 @@ void buildTiles(spg_xpbd_ctx &c, const std::vector<float4> &x, const std::vector
     hipCheck(hipStreamSynchronize(c.stream), "hipStreamSynchronize");  // the lists end here
     if (fits) {
         c.batches = std::move(plan.batches);
+        c.tileProjections = static_cast<int64_t>(plan.entries.size());
         return;
     }
     c.tileHeaders.release();
@@ -779,6 +783,24 @@ int spg_xpbd_num_launches(const spg_xpbd_ctx *ctx, int32_t *n)
 {
     if (!ctx || !n) return SPG_VBD_ERR_INVALID;
     *n = static_cast<int32_t>(ctx->launch.group_runs ? ctx->plan.size() : ctx->single.size());
+    return SPG_VBD_OK;
+}
+
+int spg_xpbd_get_substep_plan(const spg_xpbd_ctx *ctx, spg_xpbd_substep_plan *plan)
+{
+    if (!ctx || !plan) return SPG_VBD_ERR_INVALID;
+    *plan = {};
+    if (!ctx->tiled()) return spg_xpbd_num_launches(ctx, &plan->launches);
+    for (const TileBatch &b : ctx->batches) {
+        plan->launches += b.tiles ? 1 : b.groups;
+        plan->tiled_launches += b.tiles ? 1 : 0;
+        plan->tiles += b.tiles;
+    }
+    plan->tile_particles = static_cast<int64_t>(ctx->tileParticles.n);
+    plan->tile_projections = ctx->tileProjections;
+    auto bytes = [](const auto &b) { return static_cast<int64_t>(b.n * sizeof(*b.p)); };
+    plan->tile_bytes = bytes(ctx->tileRecords) + bytes(ctx->tileParticles) + bytes(ctx->tileSegments) +
+                       bytes(ctx->tileHeaders) + bytes(ctx->spare);
     return SPG_VBD_OK;
 }
 

@@ -99,6 +99,14 @@ class XpbdStats(ctypes.Structure):
         return d
 
 
+class XpbdSubstepPlan(ctypes.Structure):
+    _fields_ = [("launches", ctypes.c_int32), ("tiled_launches", ctypes.c_int32), ("tiles", ctypes.c_int64),
+                ("tile_particles", ctypes.c_int64), ("tile_projections", ctypes.c_int64), ("tile_bytes", ctypes.c_int64)]
+
+    def as_dict(self):
+        return {k: getattr(self, k) for k, _ in self._fields_}
+
+
 class ImplicitStats(ctypes.Structure):
     _fields_ = [("steps", ctypes.c_int64), ("linear_solves", ctypes.c_int64), ("cg_iterations", ctypes.c_int64),
                 ("newton_iterations", ctypes.c_int64), ("failed_substeps", ctypes.c_int64),
@@ -215,6 +223,7 @@ def vbd_lib():
         _proto(L, "spg_xpbd_num_groups", ctypes.c_int, [c, i32, i32, _ip])
         _proto(L, "spg_xpbd_get_groups", ctypes.c_int, [c, i32, i32, _ip])
         _proto(L, "spg_xpbd_num_launches", ctypes.c_int, [c, _ip])
+        _proto(L, "spg_xpbd_get_substep_plan", ctypes.c_int, [c, ctypes.POINTER(XpbdSubstepPlan)])
         _proto(L, "spg_xpbd_set_state", ctypes.c_int, [c, i32, _dp, _dp])
         _proto(L, "spg_xpbd_get_state", ctypes.c_int, [c, i32, _dp, _dp])
         _proto(L, "spg_xpbd_step", ctypes.c_int, [c, dbl, i32, _dp])
@@ -1051,6 +1060,13 @@ class XpbdContext:
         n = ctypes.c_int32(0)
         self._check(self._L.spg_xpbd_num_launches(self.h, ctypes.byref(n)))
         return n.value
+
+    def substep_plan(self):
+        """The launches of an untimed step's substep: how many, how many of them over tiles of particles, and what the
+        tiles load, project and hold."""
+        plan = XpbdSubstepPlan()
+        self._check(self._L.spg_xpbd_get_substep_plan(self.h, ctypes.byref(plan)))
+        return plan.as_dict()
 
     def state(self, obj=0):
         x, v = np.zeros((self._n[obj], 3)), np.zeros((self._n[obj], 3))

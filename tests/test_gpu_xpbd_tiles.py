@@ -39,7 +39,7 @@ SCENES = {
     "stvk cube": lambda: [scenes.cube(5, material="stvk_tet")],
     "ssnh cube": lambda: [scenes.cube(5, material="ssnh")],
     "springs": lambda: [_springs(300)],
-    "springs anywhere": lambda: [_springs(6000)],  # a tile's particles do not fit: launches per group
+    "springs anywhere": lambda: [_springs(6000)],  # most of a tile's particles lie in others
     "objects": lambda: [_cloth(20), scenes.cube(4), _springs(50), _cloth(35),
                         scenes.Scene(x=np.ones((1, 3)), x0=np.ones((1, 3)), m=np.ones(1))],
 }
@@ -86,3 +86,43 @@ def test_substep_counts(nsub):
     (x0, v0), (x1, v1) = ctx[0].state(), ctx[1].state()
     assert np.array_equal(x0, x1) and np.array_equal(v0, v1)
     assert np.abs(v1).max() > 0.1  # gravity over two frames: 0.33 m/s where the cloth falls freely
+
+
+@pytest.mark.parametrize("parallel", [True, False])
+@pytest.mark.parametrize("name", list(SCENES))
+def test_scenes_are_stepped_over_tiles(name, parallel):
+    """The scenes above do take tiles with group_runs 1, and none with group_runs 0."""
+    objs = [s.xpbd_object() for s in SCENES[name]()]
+    if not parallel and sum(len(o["x"]) for o in objs) > 3000:
+        objs = objs[:1] if len(objs) > 1 else pytest.skip("thousands of levels")
+    ctx = native.XpbdContext(objs, parallel_gauss_seidel=parallel)
+    plan, stencils = ctx.substep_plan(), sum(len(st) for o in objs for _, st, _ in o["energies"])
+    assert plan["tiled_launches"] > 0 and plan["tiles"] >= plan["tiled_launches"]
+    assert plan["launches"] <= ctx.num_launches() and plan["tile_bytes"] > 0
+    if plan["launches"] == plan["tiled_launches"]:  # everything over tiles: each stencil at least once
+        assert plan["tile_projections"] >= stencils
+        assert plan["tile_particles"] >= sum(len(o["x"]) for o in objs) * plan["tiled_launches"]
+    ctx.set_launch(group_runs=0)
+    assert ctx.substep_plan() == dict(launches=ctx.num_launches(), tiled_launches=0, tiles=0, tile_particles=0,
+                                      tile_projections=0, tile_bytes=0)
+
+
+@pytest.mark.parametrize("parallel", [True, False])
+@pytest.mark.parametrize("name", ["cloth 97", "baraff-witkin cloth", "cube 11", "stiff cube", "objects"])
+def test_runs_of_small_groups_bitwise_equal_single_launches(name, parallel):
+    """Timed steps with group_runs 1 take the small groups in runs of one workgroup (the launches of num_launches), not
+    tiles: the same state as one launch per group."""
+    objs = [s.xpbd_object() for s in SCENES[name]()]
+    if not parallel:
+        objs = objs[:1]
+    out = []
+    for runs in (0, 1):
+        ctx = native.XpbdContext(objs, parallel_gauss_seidel=parallel)
+        ctx.set_launch(group_runs=runs)
+        ctx.set_timing(True)
+        ctx.step(scenes.DT, 3, scenes.GRAVITY)
+        st = ctx.stats()
+        assert st["projection_launches"] == 3 * ctx.num_launches()
+        assert ("small_group_runs" in st["per_type"]) == (runs == 1)
+        out.append([a for o in range(len(objs)) for a in ctx.state(o)] + [st["fp64_solves"]])
+    assert all(np.array_equal(p, q) for p, q in zip(*out))
