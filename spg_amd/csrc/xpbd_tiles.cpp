@@ -13,15 +13,45 @@ namespace spgvbd {
 
 namespace {
 
-// The times the plan is chosen by, in microseconds, measured on MI355X.
-constexpr double kGroupLaunchUs = 4.4;  // one launch of one group
-constexpr double kTileLaunchUs = 5.0;   // a tile launch without its groups
-constexpr double kBytesPerUs = 5e6;     // record streaming
+// The times the plan is chosen by, in microseconds, measured on MI355X. A compute unit holds one workgroup of a tile
+// kernel at a time (its registers), so a launch of more tiles than compute units takes its time per tile several times
+// over; and each tile gathers its particles, a cache line each where they are scattered. Without these two a solid of
+// 64^3 cells took 538 tiles, whose five launches take 221 us, where its 34 groups take 152 us by themselves, and 10^6
+// particles with springs anywhere 230 us for 214. A 512x512 cloth (256 tiles): 37 us by this estimate, 33 measured;
+// 700x700 (479): 68 and 62; 1024x1024 (1024): 133 and 123.
+constexpr double kGroupLaunchUs = 4.4;    // one launch of one group, a small one
+constexpr double kGroupBytesPerUs = 4e6;  // of the records and particles of a large one
+constexpr double kTileLaunchUs = 5.0;     // a tile launch without its groups
+constexpr double kBytesPerUs = 5e6;       // record streaming and particle gathers of a tile launch
+constexpr double kParticleBytes = 64;     // of a particle that a tile loads
 constexpr int kComputeUnits = 256;
-constexpr int kPlanThreads = 8;         // host threads that build the plan
+constexpr int kPlanThreads = 8;           // host threads that build the plan
 
-// a round of one group in a tile
-double groupUs(int32_t type) { return type == 4 ? 1.6 : type <= 5 ? 1.0 : 2.5; }
+// A round of one group in a tile: steps of one launch of one round a group (a 100x100 cloth of each kind, solids of 12^3
+// and 17^3 cells) less the launch, by group.
+double groupUs(int32_t type)
+{
+    switch (type) {
+    case 4: return 1.2;
+    case 8: return 3.0;
+    case 9: return 4.5;
+    case 10: return 3.0;
+    case 11: return 1.5;
+    case 12: return 1.7;
+    case 13: return 1.5;
+    default: return 1.0;
+    }
+}
+// One group by itself. The kernels of types 8 to 10 keep an array in scratch memory: 5.5 us at 2,800 stencils, 9 at
+// 19,000, 15 at 45,000, 18 at 140,000.
+double aloneUs(const TileGroup &g)
+{
+    const double bytes = g.count * (16.0 * tilePlanes(g.type) + 32.0 * g.size);
+    const double least = g.type >= 8 && g.type <= 10 ? 5.0 + 10.0 * std::min(1.0, g.count / 40000.0) : kGroupLaunchUs;
+    return std::max(least, bytes / kGroupBytesPerUs);
+}
+// how often a compute unit takes a tile
+double waves(int64_t tiles) { return static_cast<double>((tiles + kComputeUnits - 1) / kComputeUnits); }
 
 // Bisects particles [b, e) of `order` along the longer side of their box, again and again, into `parts` ranges of equal
 // size; writes the ranges' ends to ends[0 .. parts).
@@ -73,6 +103,7 @@ struct Tiles {
 
 // Tiles of at most 256 particles, and from them tiles of up to twice and four times as many: the halves and quarters
 // of a tile are consecutive.
+constexpr int64_t kLargeTile = 1024;
 std::array<Tiles, 3> makeTiles(const float *xyz, int stride, const std::vector<int64_t> &objects)
 {
     std::array<Tiles, 3> out;
@@ -82,20 +113,20 @@ std::array<Tiles, 3> makeTiles(const float *xyz, int stride, const std::vector<i
     for (size_t o = 0; o + 1 < objects.size(); ++o) {
         const int64_t n = objects[o + 1] - objects[o];
         if (n == 0) continue;
-        const int64_t large = (n + 1023) / 1024;
+        const int64_t large = (n + kLargeTile - 1) / kLargeTile;
         std::vector<int64_t> ends(large);
         bisect(xyz, stride, order.data(), objects[o], objects[o + 1], large, ends.data());
         int64_t b = objects[o];
         for (int64_t e : ends) {
             out[2].ends.push_back(e);
             // an object of one tile may be much smaller than 1024 particles
-            const int64_t halves = e - b > 512 ? 2 : 1;
+            const int64_t halves = e - b > kLargeTile / 2 ? 2 : 1;
             std::vector<int64_t> half(halves);
             bisect(xyz, stride, order.data(), b, e, halves, half.data());
             int64_t c = b;
             for (int64_t f : half) {
                 out[1].ends.push_back(f);
-                const int64_t quarters = f - c > 256 ? 2 : 1;
+                const int64_t quarters = f - c > kLargeTile / 4 ? 2 : 1;
                 std::vector<int64_t> quarter(quarters);
                 bisect(xyz, stride, order.data(), c, f, quarters, quarter.data());
                 out[0].ends.insert(out[0].ends.end(), quarter.begin(), quarter.end());
@@ -201,10 +232,8 @@ std::vector<TileBatch> cut(const Tiles &tiles, const Holders &holders, const std
     constexpr int kSamples = 5;
     const int64_t nt = tiles.count(), ns = std::min<int64_t>(nt, kSamples);
     std::vector<Grower> grower(ns, Grower(holders, groups));
-    // rounds of the largest tile, or of the whole chip where the tiles outnumber it
-    auto groupCost = [&](int32_t g, double largest, double total) {
-        const double rounds = std::max(std::ceil(largest / threads), total / (double(threads) * kComputeUnits));
-        return groupUs(groups[g].type) * std::max(1.0, rounds);
+    auto groupCost = [&](int32_t g, double stencils) {  // of a tile's stencils of the group
+        return waves(nt) * groupUs(groups[g].type) * std::max(1.0, std::ceil(stencils / threads));
     };
     std::vector<TileBatch> out;
     std::vector<int32_t> list;
@@ -215,7 +244,7 @@ std::vector<TileBatch> cut(const Tiles &tiles, const Holders &holders, const std
             grower[k].start(tiles.begin(t), tiles.size(t));
         }
         int32_t first = last + 1;
-        double compute = 0.0, bytes = 0.0;
+        double compute = 0.0, bytes = 0.0, loads = 0.0;
         while (first > 0 && last - first + 1 < kTileMaxGroups) {
             const int32_t g = first - 1;
             double largest = 0.0, total = 0.0;
@@ -225,15 +254,19 @@ std::vector<TileBatch> cut(const Tiles &tiles, const Holders &holders, const std
                 largest = std::max<double>(largest, list.size());
                 total += static_cast<double>(list.size()) * nt / ns;
             }
-            const double with = groupCost(g, largest, total), alone = groupCost(g, 0.0, groups[g].count);
-            if (!fits || (first <= last && with - alone > kTileLaunchUs)) break;
+            const double with = groupCost(g, largest), without = groupCost(g, static_cast<double>(groups[g].count) / nt);
+            if (!fits || (first <= last && with - without > kTileLaunchUs)) break;
             compute += with;
             bytes += total * 16.0 * tilePlanes(groups[g].type);
+            loads = 0.0;
+            for (int64_t k = 0; k < ns; ++k) loads += static_cast<double>(grower[k].particles.size()) * nt / ns;
             first = g;
         }
         const int32_t count = std::max(1, last - first + 1);
         first = last - count + 1;
-        const double tile = kTileLaunchUs + std::max(compute, bytes / kBytesPerUs), separate = kGroupLaunchUs * count;
+        const double tile = kTileLaunchUs + std::max(compute, bytes / kBytesPerUs) + loads * kParticleBytes / kBytesPerUs;
+        double separate = 0.0;
+        for (int32_t g = first; g <= last; ++g) separate += aloneUs(groups[g]);
         const bool use = count > 1 && tile < separate;
         us += use ? tile : separate;
         out.push_back({first, count, 0, use ? static_cast<int32_t>(nt) : 0, 0});
@@ -330,6 +363,16 @@ TilePlan buildTilePlan(const float *xyz, int stride, const std::vector<int64_t> 
     const int64_t nv = objects.back();
     if (nv == 0 || groups.size() < 2) return {};
     if (nv * static_cast<int64_t>(groups.size()) > kHoldersMax) return {};
+    // with so many tiles, the largest there are, that no group is faster in a tile than by itself there is nothing to plan
+    int64_t fewest = 0;
+    for (size_t o = 0; o + 1 < objects.size(); ++o) fewest += (objects[o + 1] - objects[o] + kLargeTile - 1) / kLargeTile;
+    double alone = 0.0;
+    bool any = false;
+    for (const auto &g : groups) {
+        alone += aloneUs(g);
+        any |= waves(fewest) * groupUs(g.type) < aloneUs(g);
+    }
+    if (!any) return {};
     std::vector<std::vector<int32_t>> stencilsOf(groups.size());
     forAll(groups.size(), kPlanThreads, [&](int64_t g) {
         stencilsOf[g].resize(static_cast<size_t>(groups[g].count) * groups[g].size);
@@ -348,8 +391,13 @@ TilePlan buildTilePlan(const float *xyz, int stride, const std::vector<int64_t> 
             }
             batches[k] = cut(tiles[k], holders, groups, threads, margin, us[k]);
         });
-        const size_t best = std::min_element(us.begin(), us.end()) - us.begin();
-        if (us[best] >= kGroupLaunchUs * static_cast<double>(groups.size())) return {};
+        // larger tiles where they are 2% faster: the smaller ones use more of the chip (17^3-cell solid: 24 tiles 60 us, 12
+        // tiles 62, by the estimate 63.4 and 62.7)
+        size_t best = 0;
+        for (size_t k = 1; k < us.size(); ++k)
+            if (us[k] < 0.98 * us[best]) best = k;
+        const bool tiled = std::any_of(batches[best].begin(), batches[best].end(), [](const TileBatch &b) { return b.tiles > 0; });
+        if (!tiled || us[best] >= alone) return {};
         Tiles &t = tiles[best];
         int64_t b = 0;
         for (int64_t e : t.ends) {  // ascending within a tile: its particles are then mostly consecutive in memory

@@ -29,3 +29,14 @@ def test_plan_equals_one_launch_per_group(check, kind, size, serial, threads):
     assert out.returncode == 0, out.stdout
     if kind != "net" and size > 2:
         assert not out.stdout.startswith("batches 0"), out.stdout
+
+
+# one launch takes as long as its workgroups follow each other on a compute unit: 256 tiles at a time on 256 of them
+@pytest.mark.parametrize("kind,size,threads,tiled", [("cloth", 512, 1024, True), ("cloth", 1024, 1024, True), ("cube", 17, 512, True),
+                                                     ("cube", 48, 512, True), ("cube", 64, 512, False)])
+def test_tiles_where_they_are_faster(check, kind, size, threads, tiled):
+    """Measured, a substep in tiles and with a launch per group, us: cloths 33 and 84, 125 and 182; solids 60 and 91, 84 and
+    128, and 221 and 152 where 64^3 cells are cut into 538 tiles."""
+    out = subprocess.run([check, kind, str(size), "0", str(threads)], capture_output=True, text=True)
+    assert out.returncode == 0, out.stdout
+    assert (int(out.stdout.split()[3]) > 0) == tiled, out.stdout
