@@ -230,7 +230,7 @@ struct spg_implicit_ctx {
             copy(v0.p, v.p);
             assemble(x.p, true);
             // rhs = dt (f + dt K v0) with K = -H
-            hipCheck(launchSymSpmv(sym(H.p), v0.p, -1.0, tmp.p, nullptr, stream), "spmv launch");
+            hipCheck(launchSymSpmv(sym(H.p), v0.p, -1.0, tmp.p, stream), "spmv launch");
             lin(rhs.p, 1.0, f.p, dt, tmp.p);
             lin(rhs.p, dt, rhs.p);
             solve(1.0, dt * dt, rhs.p, dv.p, tol, maxIt);
@@ -270,7 +270,7 @@ struct spg_implicit_ctx {
             assemble(x.p, true);
             // w = x0 - x_{-1} + 2 dt v0; tmp = K w = -H w
             lin(rhs.p, 1.0, x0.p, -1.0, xm1.p, 2 * dt, v0.p);
-            hipCheck(launchSymSpmv(sym(H.p), rhs.p, -1.0, tmp.p, nullptr, stream), "spmv launch");
+            hipCheck(launchSymSpmv(sym(H.p), rhs.p, -1.0, tmp.p, stream), "spmv launch");
             // tmp = 2/3 dt (f + 1/3 K w); rhs = 1/3 M (v0 - v_{-1}) + tmp
             lin(tmp.p, 2.0 / 3.0 * dt, f.p, 2.0 / 3.0 * dt / 3.0, tmp.p);
             lin(dv.p, 1.0, v0.p, -1.0, vm1.p);
@@ -583,7 +583,8 @@ void buildContext(spg_implicit_ctx &c, const spg_vbd_object *objs, int32_t nObje
     c.H.alloc(9 * c.nUpper);
     c.A.alloc(9 * c.nUpper);
     c.invdiag.alloc(c.ndof);
-    for (auto *b : {&c.cgr, &c.cgz, &c.cgp, &c.cgq, &c.x0, &c.v0, &c.vi, &c.dv, &c.rhs, &c.tmp, &c.xm1, &c.vm1})
+    if (cgInTwoKernels(c.spmvBytes(), c.ndof)) c.cgz.alloc(c.ndof);
+    for (auto *b : {&c.cgr, &c.cgp, &c.cgq, &c.x0, &c.v0, &c.vi, &c.dv, &c.rhs, &c.tmp, &c.xm1, &c.vm1})
         b->alloc(c.ndof);
     c.partial.alloc(std::max<int64_t>(2 * kCgBlocks, spmvPartials(c.np)));
     c.partial2.alloc(2 * kCgBlocks);
@@ -826,10 +827,10 @@ int spg_implicit_bench_spmv(spg_implicit_ctx *ctx, double alpha, double beta, in
         hipCheck(launchCombine(ctx->nUpper, ctx->H.p, -beta, ctx->np, ctx->upPtr.p, ctx->mass.p, alpha, ctx->A.p,
                                ctx->stream),
                  "combine launch");
-        hipCheck(launchSymSpmv(ctx->sym(ctx->A.p), ctx->v.p, 1.0, ctx->tmp.p, nullptr, ctx->stream), "spmv launch");
+        hipCheck(launchSymSpmv(ctx->sym(ctx->A.p), ctx->v.p, 1.0, ctx->tmp.p, ctx->stream), "spmv launch");
         hipCheck(hipEventRecord(ctx->ev0, ctx->stream), "hipEventRecord");
         for (int32_t r = 0; r < repeats; ++r)
-            hipCheck(launchSymSpmv(ctx->sym(ctx->A.p), ctx->v.p, 1.0, ctx->tmp.p, nullptr, ctx->stream),
+            hipCheck(launchSymSpmv(ctx->sym(ctx->A.p), ctx->v.p, 1.0, ctx->tmp.p, ctx->stream),
                      "spmv launch");
         hipCheck(hipEventRecord(ctx->ev1, ctx->stream), "hipEventRecord");
         hipCheck(hipEventSynchronize(ctx->ev1), "hipEventSynchronize");

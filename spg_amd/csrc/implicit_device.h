@@ -62,9 +62,9 @@ hipError_t launchAssembleHessian(int64_t nUpper, const int32_t *upRow, const int
 // of (i, i))
 hipError_t launchCombine(int64_t nBlocks, const double *H, double c, int64_t nParticles, const int64_t *diagBlock,
                          const double *mass, double a, double *A, hipStream_t stream);
-// y = s * (A x) for the symmetric block matrix; partial (may be null): per-workgroup partial sums of
-// x . y, spmvPartials(rows) of them
-hipError_t launchSymSpmv(const SymBsr &A, const double *x, double s, double *y, double *partial, hipStream_t stream);
+// y = s * (A x) for the symmetric block matrix
+hipError_t launchSymSpmv(const SymBsr &A, const double *x, double s, double *y, hipStream_t stream);
+// partial sums of x . y that a product of the conjugate gradient leaves, at most
 int spmvPartials(int64_t rows);
 // the full block rows of s * A (rowPtr/col: the full pattern, diagBlock: index of (i, i) in it) into out
 hipError_t launchExpandSym(const SymBsr &A, double s, const int64_t *rowPtr, const int32_t *col,
@@ -81,12 +81,17 @@ struct CgScalars {
 constexpr int kCgBlocks = 512;  // workgroups of the vector kernels (fixed: deterministic reductions)
 // a CG needs two partial-sum buffers: pPartial of max(2 kCgBlocks, spmvPartials(rows)) doubles (also used
 // by launchCgInit) and uPartial of 2 kCgBlocks
+// Whether an iteration takes two kernels (figures at cgProductKernel): where the product's bytes and the six vectors stay
+// under three quarters of the 256 MB of the Infinity Cache.
+inline bool cgInTwoKernels(double productBytes, int64_t n) { return productBytes + 48.0 * n < 201326592.0; }
+// z null: an iteration takes three kernels
 hipError_t launchCgInit(int64_t n, const double *b, const double *invdiag, double *x, double *r, double *z, double *p,
                         double *q, double *partial, CgScalars *s, double tol, hipStream_t stream);
-// iteration `iteration` (0-based, launch order) in two kernels: the convergence test and beta of the one before,
-// p = z + beta p, q = A z + beta q (= A p); alpha, x += alpha p, r -= alpha q, z = D^-1 r. The last one of the budget is
-// followed by its own test. Non-null events are recorded right before and after the first kernel (to time the product
-// inside a solve).
+// iteration `iteration` (0-based, launch order). In two kernels: the convergence test and beta of the one before,
+// p = z + beta p, q = A z + beta q (= A p); alpha, x += alpha p, r -= alpha q, z = D^-1 r. In three (z null): q = A p;
+// alpha, x += alpha p, r -= alpha q; the convergence test and beta, p = D^-1 r + beta p. The last one of the budget ends
+// with its test. Non-null events are recorded right before and after the first kernel (to time the product inside a
+// solve).
 hipError_t launchCgIteration(const SymBsr &A, int64_t n, const double *invdiag, double *x, double *r, double *z,
                              double *p, double *q, double *pPartial, double *uPartial, CgScalars *s, int32_t maxIters,
                              int32_t iteration, hipStream_t stream, hipEvent_t spmvStart = nullptr,

@@ -259,10 +259,13 @@ __device__ __forceinline__ void store3(double *__restrict__ v, int64_t j, V3<dou
     v[3 * j + 2] = a.z;
 }
 
+// cg (may be null): the solve whose iteration `iteration` the product belongs to; nothing is done once it has ended.
 __global__ void __launch_bounds__(kSpmvBlock) symSpmvKernel(SymBsr A, const double *__restrict__ x, double s,
-                                                           double *__restrict__ y, double *__restrict__ partial)
+                                                           double *__restrict__ y, double *__restrict__ partial,
+                                                           const CgScalars *cg, int32_t iteration)
 {
     __shared__ double sh[kSpmvBlock / 64];
+    if (cg && cg->last < iteration) return;
     const int32_t blk = xcdContiguous(static_cast<int32_t>(blockIdx.x), static_cast<int32_t>(gridDim.x));
     const int64_t t = blk * static_cast<int64_t>(kSpmvBlock) + threadIdx.x;
     const int64_t row = t / kSpmvG;
@@ -335,6 +338,7 @@ __global__ void __launch_bounds__(256) cgInitKernel(int64_t n, const double *__r
                                                     double *__restrict__ p, double *__restrict__ q,
                                                     double *__restrict__ partial)
 {
+    // z null: an iteration in three kernels, whose first direction this is
     __shared__ double sh[4];
     const int64_t chunk = (n + gridDim.x - 1) / gridDim.x;
     const int64_t b0 = blockIdx.x * chunk, e0 = b0 + chunk < n ? b0 + chunk : n;
@@ -342,8 +346,10 @@ __global__ void __launch_bounds__(256) cgInitKernel(int64_t n, const double *__r
         const double bi = b[i];
         x[i] = 0.0;
         r[i] = bi;
-        z[i] = invdiag[i] * bi;
-        p[i] = 0.0;
+        const double zi = invdiag[i] * bi;
+        p[i] = z ? 0.0 : zi;
+        if (!z) continue;
+        z[i] = zi;
         q[i] = 0.0;
     }
     const double bb = chunkSum(n, [&](int64_t i) { return b[i] * b[i]; }, sh);
@@ -467,20 +473,24 @@ __device__ __forceinline__ bool cgNext(CgScalars *s, double rr, double rz, doubl
     return true;
 }
 
-// An iteration in two kernels. The first closes the iteration before (convergence, beta) and forms p = z + beta p and
-// q = A p = A z + beta q, z = D^-1 r: the product is taken of z, which the kernel before left whole, so no kernel in
-// between has to form p for the gather, and its loads do not wait for beta. The second (cgUpdateKernel) takes alpha and
-// updates x, r and z. Every workgroup adds up the partial sums itself, in the same order, and loads its first entries
-// before that.
+// An iteration in two kernels, for systems that the caches hold (cgInTwoKernels). The first closes the iteration before
+// (convergence, beta) and forms p = z + beta p and q = A p = A z + beta q, z = D^-1 r: the product is taken of z, which the
+// kernel before left whole, so no kernel in between has to form p for the gather, and its loads do not wait for beta. The
+// second (cgUpdateKernel) takes alpha and updates x, r and z. Every workgroup adds up the partial sums itself, in the same
+// order, and loads its first entries before that.
 //
 // What bounds an iteration: at 200x200 particles the latency of two dependent launches with a reduction each (the matrix,
-// 20 MB, comes from the L2s; the product takes 10.1 us of the 15.8, 8.1 by itself), at 512x512 the 0.13 GB of the matrix.
-// In three kernels (product, update, direction p = z + beta p), whose sums waited for each other through shuffles, an
-// iteration took 22.4 us at 48x48 particles, 18.7 at 100x100, 21.9 at 200x200, 37.0 at 330x330 and 61.4 at 512x512; now
-// 14.4, 11.5, 15.8, 31.2 and 59.3. Of that the sums by lane permutations are 2 to 3 us, workgroups of 512 instead of 1024
-// threads 1.5 (the barrier waits for fewer). Forming p in the gather (z + beta p of every neighbour) took 19.2, 15.7, 21,
-// 38 and 70. The recurrence for q costs no accuracy: after 1517 iterations at 200x200 particles b - A x is 9.7347e-11 |b|
-// and the r that was carried along 9.7350e-11 |b| (9.7229e-11 and 9.7228e-11 with q = A p).
+// 20 MB, comes from the L2s; the product takes 12.5 us of the 17.4, 8.2 by itself), from 500x500 on the memory. Cloths of
+// n x n particles, us an iteration, in two kernels and in three (product, update, direction p = D^-1 r + beta p):
+//    48: 12.9  17.8    200: 17.4  20.5    330: 30.8  32.6    420: 41.9  43.5    480: 52.4  53.5    512: 55.4  54.0
+//   570: 67.0  64.5    700:  123   115    850:  185   175   1000:  253   235   1200:  362   333
+// Beyond the caches p and q, read and written by one lane of eight at the end of a product, cost more than the passes over
+// the vectors that they save. Of what two kernels gain where they do, the sums by lane permutations are 2 to 3 us,
+// workgroups of 512 instead of 1024 threads 1.5 (the barrier waits for fewer). With sums through shuffles that waited for each
+// other three kernels took 20.8 us at 48x48, 23.5 at 200x200, 57.2 at 512x512 and 239 at 1000x1000. Forming p in the gather
+// (z + beta p of every neighbour) took 4 to 11 us more than q's recurrence, which costs little accuracy: after 1517 iterations
+// at 200x200 particles b - A x is 9.7347e-11 |b| and the r that was carried along 9.7350e-11 |b| (9.7229e-11 and 9.7228e-11
+// with q = A p).
 constexpr int kCgProductBlock = 512;
 __global__ void __launch_bounds__(kCgProductBlock) cgProductKernel(SymBsr A, const double *__restrict__ z,
                                                               double *__restrict__ p, double *__restrict__ q,
@@ -533,8 +543,9 @@ __global__ void __launch_bounds__(kCgProductBlock) cgProductKernel(SymBsr A, con
 
 // alpha = r.z / p.q, x += alpha p, r -= alpha q, z = D^-1 r; partial sums of r.r and r.z. Workgroups take contiguous
 // chunks of the vectors, renumbered so that each XCD's chunks are the rows whose products it forms: what one kernel
-// writes the next finds in the same L2.
+// writes the next finds in the same L2. TWO: of an iteration in two kernels, which reads z again.
 constexpr int kCgAhead = 4;  // entries of a thread loaded together
+template <bool TWO>
 __global__ void __launch_bounds__(256) cgUpdateKernel(int64_t n, const double *__restrict__ invdiag,
                                                       double *__restrict__ x, double *__restrict__ r,
                                                       double *__restrict__ z, const double *__restrict__ p,
@@ -578,7 +589,7 @@ __global__ void __launch_bounds__(256) cgUpdateKernel(int64_t n, const double *_
                 const double ri = rv[k] - alpha * qv[k], zi = dv[k] * ri;
                 x[i] = xv[k] + alpha * pv[k];
                 r[i] = ri;
-                z[i] = zi;
+                if constexpr (TWO) z[i] = zi;
                 rr += ri * ri;
                 rz += ri * zi;
             }
@@ -587,6 +598,47 @@ __global__ void __launch_bounds__(256) cgUpdateKernel(int64_t n, const double *_
         load(i0);
     }
     storeBlockSums<4>(rr, rz, sh, partial + blockIdx.x, partial + gridDim.x + blockIdx.x);
+}
+
+// The third kernel of an iteration in three: its end (convergence, beta) and p = D^-1 r + beta p.
+__global__ void __launch_bounds__(256) cgDirectionKernel(int64_t n, const double *__restrict__ invdiag,
+                                                         const double *__restrict__ r, double *__restrict__ p,
+                                                         const double *__restrict__ uPartial, int nbU, CgScalars *s,
+                                                         int32_t iteration)
+{
+    __shared__ double sh[8];
+    const int32_t last = s->last;
+    const double before = s->absNew[iteration & 1], threshold = s->threshold;
+    const int64_t chunk = (n + gridDim.x - 1) / gridDim.x;
+    const int64_t b0 = xcdContiguous(blockIdx.x, gridDim.x) * chunk, e0 = b0 + chunk < n ? b0 + chunk : n;
+    double pv[kCgAhead], rv[kCgAhead], dv[kCgAhead];
+    const auto load = [&](int64_t i0) {
+#pragma unroll
+        for (int k = 0; k < kCgAhead; ++k) {
+            const int64_t i = i0 + k * 256;
+            if (i < e0) {
+                pv[k] = p[i];
+                rv[k] = r[i];
+                dv[k] = invdiag[i];
+            }
+        }
+    };
+    int64_t i0 = b0 + threadIdx.x;
+    load(i0);
+    double u, v, rr, rz, beta;
+    threadTotals<4>(uPartial, uPartial + nbU, nbU, u, v);
+    if (last < iteration) return;  // `iteration` at the least while this kernel may store it
+    blockTotals<4>(u, v, sh, rr, rz);
+    if (!cgNext(s, rr, rz, before, threshold, iteration + 1, blockIdx.x == 0 && threadIdx.x == 0, beta)) return;
+    while (i0 < e0) {
+#pragma unroll
+        for (int k = 0; k < kCgAhead; ++k) {
+            const int64_t i = i0 + k * 256;
+            if (i < e0) p[i] = dv[k] * rv[k] + beta * pv[k];
+        }
+        i0 += kCgAhead * 256;
+        load(i0);
+    }
 }
 
 // After the last iteration of the budget: its convergence test (x is the last iterate either way).
@@ -732,10 +784,10 @@ int spmvGrid(int64_t rows) { return blocksFor(rows * kSpmvG, kSpmvBlock); }
 int cgProductGrid(int64_t rows) { return blocksFor(rows * kSpmvG, kCgProductBlock); }
 int spmvPartials(int64_t rows) { return std::max(spmvGrid(rows), cgProductGrid(rows)); }
 
-hipError_t launchSymSpmv(const SymBsr &A, const double *x, double s, double *y, double *partial, hipStream_t stream)
+hipError_t launchSymSpmv(const SymBsr &A, const double *x, double s, double *y, hipStream_t stream)
 {
     if (A.rows <= 0) return hipSuccess;
-    symSpmvKernel<<<spmvGrid(A.rows), kSpmvBlock, 0, stream>>>(A, x, s, y, partial);
+    symSpmvKernel<<<spmvGrid(A.rows), kSpmvBlock, 0, stream>>>(A, x, s, y, nullptr, nullptr, 0);
     return hipGetLastError();
 }
 
@@ -763,14 +815,21 @@ hipError_t launchCgIteration(const SymBsr &A, int64_t n, const double *invdiag, 
         const hipError_t e = hipEventRecord(spmvStart, stream);
         if (e != hipSuccess) return e;
     }
-    const int grid = cgProductGrid(A.rows);
-    cgProductKernel<<<grid, kCgProductBlock, 0, stream>>>(A, z, p, q, uPartial, pPartial, s, iteration);
+    const int grid = z ? cgProductGrid(A.rows) : spmvGrid(A.rows);
+    if (z)
+        cgProductKernel<<<grid, kCgProductBlock, 0, stream>>>(A, z, p, q, uPartial, pPartial, s, iteration);
+    else
+        symSpmvKernel<<<grid, kSpmvBlock, 0, stream>>>(A, p, 1.0, q, pPartial, s, iteration);
     if (spmvEnd) {
         const hipError_t e = hipEventRecord(spmvEnd, stream);
         if (e != hipSuccess) return e;
     }
-    cgUpdateKernel<<<kCgBlocks, 256, 0, stream>>>(n, invdiag, x, r, z, p, q, pPartial, grid, uPartial, s, iteration);
-    if (iteration + 1 == maxIters) cgFinishKernel<<<1, 256, 0, stream>>>(uPartial, kCgBlocks, s, maxIters);
+    const auto update = z ? cgUpdateKernel<true> : cgUpdateKernel<false>;
+    update<<<kCgBlocks, 256, 0, stream>>>(n, invdiag, x, r, z, p, q, pPartial, grid, uPartial, s, iteration);
+    if (iteration + 1 == maxIters)
+        cgFinishKernel<<<1, 256, 0, stream>>>(uPartial, kCgBlocks, s, maxIters);
+    else if (!z)
+        cgDirectionKernel<<<kCgBlocks, 256, 0, stream>>>(n, invdiag, r, p, uPartial, kCgBlocks, s, iteration);
     return hipGetLastError();
 }
 

@@ -61,3 +61,30 @@ def test_zero_right_hand_side(system):
     ctx, A, b, h = system
     x, it, err = ctx.cg_solve(1.0, -h * h, np.zeros_like(b))
     assert it == 0 and err == 0 and not x.any()
+
+
+@pytest.fixture(scope="module")
+def large_system():
+    """A cloth whose matrix and vectors the caches do not hold: an iteration takes three kernels instead of two. beta is such
+    that no row of beta K sums to more than 0.9 of the mass: by Gershgorin the eigenvalues of M + beta K lie between 0.1 and
+    1.9 of the mass, the condition number is below 19, and 1e-9 is far above what the summation order can do."""
+    import scipy.sparse as sp
+    s = scenes.cloth(520, young=1e3, pin="top_row", noise=1e-4)
+    ctx = native.ImplicitContext([s.vbd_object()], "baraff_witkin")
+    assert ctx.spmv_bytes() + 48 * ctx.num_dofs() > 201326592
+    K = ctx.stiffness()
+    beta = -0.9 * s.m[0] / abs(K).sum(axis=1).max()
+    A = (sp.diags(np.repeat(s.m, 3)) + beta * K).tocsr()
+    b = scenes.DT * ctx.system_force(s.gravity) + 1e-3 * np.random.default_rng(4).standard_normal(3 * s.n)
+    return ctx, A, b, beta
+
+
+@pytest.mark.parametrize("budget,tol", [(0, 1e-6), (1, 1e-6), (2, 1e-6), (7, 1e-9), (8, 1e-9), (9, 1e-9), (17, 1e-12), (300, 1e-2),
+                                        (300, 1e-3), (300, 1e-4), (300, 1e-8), (300, 10.0)])
+def test_iterates_and_counts_of_a_large_system(large_system, budget, tol):
+    ctx, A, b, beta = large_system
+    x, it, err = ctx.cg_solve(1.0, beta, b, tol=tol, max_iters=budget)
+    ex, eit, eerr = _reference(A, b, tol, budget)
+    assert it == eit
+    assert np.linalg.norm(x - ex) <= 1e-9 * max(np.linalg.norm(ex), 1e-300)
+    assert err == pytest.approx(eerr, rel=1e-5, abs=1e-14)
