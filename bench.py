@@ -20,8 +20,9 @@ learned    = time to a 1e-4 relative FP64 force residual, learned warm start vs 
              cloth (network trained in this run on the GPU from 256 config-4-style cloths)
 batched    = 256-cloth batch (config 4) throughput, one launch per colour for all instances
 volumetric = 64^3-cell Stable Neo-Hookean cube (config 3) throughput
-xpbd       = the XPBD parallel Gauss-Seidel step (spg's XPBD(true)) on the same cloth: stencil projections/s,
-             per-type projection-kernel rooflines, and the FP64 oracle's XPBD step on the host cores
+xpbd       = the XPBD parallel Gauss-Seidel step (spg's XPBD(true)) on the same cloth: stencil projections/s, the
+             roofline of the tile kernel that these steps run, per-type rooflines of the kernels of one stencil
+             group (timed steps run those), and the FP64 oracle's XPBD step on the host cores
 further_energies = VBD on the same cloth built from the further energies (Baraff-Witkin membrane and bending,
              continuum edge springs), and the oracle's step (one iteration) on the same cloth on the host cores
 rigid_bodies = VBD on rigid bodies (FP64 6x6 blocks) on a 512x512 lattice of boxes joined by springs and
@@ -30,9 +31,12 @@ implicit   = the Baraff-Witkin implicit Euler step (FP64: element Hessians, bloc
              the reference's 1e-5 / 300-iteration settings) on the same cloth, the roofline of the symmetric
              block-sparse SpMV sampled inside the CG, and the oracle's step on a 128x128 cloth on the host cores
 
+The last line on stdout is one short JSON object: the contract's fields, the roofline, the CPU baseline and each
+section's value. Everything measured goes to the file --record (bench_record.json beside this script).
+
 Usage: python bench.py [--gpus 1] [--steps 200] [--warmup 10] [--seed 3] [--no-cpu] [--no-learned]
                        [--no-batched] [--no-volumetric] [--no-xpbd] [--xpbd-substeps 20] [--no-implicit]
-                       [--no-rigid] [--rigid-n 512]
+                       [--no-rigid] [--rigid-n 512] [--record FILE]
 """
 import argparse
 import json
@@ -71,6 +75,7 @@ def main():
     ap.add_argument("--no-rigid", action="store_true", help="skip the rigid-body VBD measurement")
     ap.add_argument("--rigid-n", type=int, default=512, help="side of the rigid-body lattice")
     ap.add_argument("--implicit-steps", type=int, default=4, help="timed Baraff-Witkin steps")
+    ap.add_argument("--record", default=os.path.join(ROOT, "bench_record.json"), help="file for the full record")
     ap.add_argument("--copy-calibration", type=int, default=0, metavar="BYTES",
                     help="only run the plain copy kernel of BYTES (counter calibration) and exit")
     ap.add_argument("--barrier-calibration", action="store_true",
@@ -241,7 +246,29 @@ def main():
         "implicit": implicit,
         "rigid_bodies": rigid,
     }
-    print(json.dumps(out))
+    try:
+        with open(args.record, "w") as f:
+            json.dump(out, f, indent=1)
+    except OSError as e:
+        print(f"# the full record was not written: {e}", file=sys.stderr, flush=True)
+    print(json.dumps(summary(out)), flush=True)
+
+
+def summary(out):
+    """The record's short form: what a reader of the last line needs, within 2,000 characters (the learned comparison's lists
+    alone are ten times as long)."""
+    def pick(d, *keys):
+        return None if d is None else {k: (float(f"{d[k]:.6g}") if isinstance(d[k], float) else d[k]) for k in keys if k in d}
+
+    line = {k: out[k] for k in ("metric", "value", "unit", "n_gpus", "steps", "warmup", "ms_per_step", "higher_is_better",
+                                "scaling", "vs_baseline", "dtype", "data")}
+    line["config"] = pick(out["config"], "workload", "launch")
+    line["roofline"] = pick(out["roofline"], "bound", "kernel", "achieved", "peak", "unit", "frac", "traffic", "mean_launch_us")
+    line["cpu_baseline"] = pick(out["cpu_baseline"], "value", "unit", "cores", "kind", "one_core_value", "ad_mode_value")
+    line["learned"] = pick(out["learned"], "plain_ms", "learned_ms", "time_ratio", "iteration_ratio", "all_converged")
+    for k in ("batched", "volumetric", "further_energies", "xpbd", "implicit", "rigid_bodies"):
+        line[k] = pick(out[k], "value", "unit", "ms_per_step")
+    return line
 
 
 def _throughput(scene_list, steps):
@@ -420,10 +447,11 @@ def rigid_throughput(args, steps=20):
 
 
 def xpbd_throughput(scene, args):
-    """XPBD(true) on the bench's cloth: each step is args.xpbd_substeps substeps of one projection of every
-    stencil, in stencil-colour launches (14 bending + 7 membrane + 1 anchor per substep), captured in a
-    hipGraph; every step starts from the initial state. Roofline per projection kernel type from an
-    event-timed step right after the throughput region."""
+    """XPBD(true) on the bench's cloth: each step is args.xpbd_substeps substeps of one projection of every stencil,
+    captured in a hipGraph, a substep in the launches of its plan (over tiles of particles); every step starts from the
+    initial state. Roofline of the tile kernel from the same steps: the compulsory bytes of a substep (each stencil's tile
+    record once, each particle read and written once) over the time that one more substep takes. Timed steps launch the
+    stencil groups one by one: their section's times are those kernels', not the throughput region's."""
     import numpy as np
     from spg_amd import native
 
@@ -434,16 +462,22 @@ def xpbd_throughput(scene, args):
     ctx.set_launch(use_graph=1, block_size=256)
     n_st = sum(len(st) for _, st, _ in scene.energies)
     ctx.save_state()
-    for _ in range(3):
-        ctx.restore_state()
-        ctx.step(scene.dt, nsub, scene.gravity)
-    ctx.synchronize()
-    t0 = time.perf_counter()
-    for _ in range(steps):
-        ctx.restore_state()
-        ctx.step(scene.dt, nsub, scene.gravity)
-    ctx.synchronize()
-    wall = time.perf_counter() - t0
+
+    def run(substeps):
+        for _ in range(3):
+            ctx.restore_state()
+            ctx.step(scene.dt, substeps, scene.gravity)
+        ctx.synchronize()
+        t0 = time.perf_counter()
+        for _ in range(steps):
+            ctx.restore_state()
+            ctx.step(scene.dt, substeps, scene.gravity)
+        ctx.synchronize()
+        return time.perf_counter() - t0
+
+    wall = run(nsub)
+    substep_us = (run(2 * nsub) - wall) / (steps * nsub) * 1e6
+    plan = ctx.substep_plan()
     ctx.reset_stats()
     ctx.set_timing(True)
     ctx.restore_state()
@@ -459,14 +493,26 @@ def xpbd_throughput(scene, args):
         per_type[k] = {"launches": d["launches"], "mean_launch_us": ms * 1e3, "achieved_GBs": gbs,
                        "frac": gbs / HBM_PEAK_GBS, "bytes_per_launch": d["bytes"] / d["launches"]}
     dom = max(per_type, key=lambda k: st["per_type"][k]["ms"])
+    record = {"stvk": 48, "bending": 16, "anchor": 32}  # bytes of a stencil's tile record
+    substep_bytes = sum(record[k] * len(s) for k, s, _ in scene.energies) + 32 * scene.n
+    achieved = substep_bytes / (substep_us * 1e-6) / 1e9
     out = {"workload": f"same cloth, XPBD parallel Gauss-Seidel, dt=1/60, {nsub} substeps/step, "
-                       f"{ctx.num_launches()} projection launches per substep, hipGraph replay",
+                       f"{plan['launches']} projection launches per substep ({plan['tiled_launches']} over "
+                       f"{plan['tiles']} tiles), hipGraph replay",
            "value": n_st * nsub * steps / wall, "unit": "stencil-projections/s",
            "ms_per_step": wall * 1e3 / steps, "steps": steps, "substeps": nsub, "stencils": n_st,
-           "projection_ms_per_substep": st["projection_ms"] / nsub,
-           "roofline": {"bound": "hbm", "kernel": f"xpbdProjectKernel<{dom}>", "achieved": per_type[dom]["achieved_GBs"],
-                        "peak": HBM_PEAK_GBS, "unit": "GB/s", "frac": per_type[dom]["frac"]},
-           "per_type": per_type, "fp64_solves": st["fp64_solves"], "setup_s": setup, "state_finite": finite}
+           "substep_us": substep_us, "substep_plan": plan,
+           "roofline": {"bound": "latency of the chain of stencil groups in a tile", "kernel": "xpbdTileKernel",
+                        "achieved": achieved, "peak": HBM_PEAK_GBS, "unit": "GB/s", "frac": achieved / HBM_PEAK_GBS,
+                        "algorithmic_bytes_per_substep": substep_bytes} if plan["tiled_launches"] else None,
+           "launches_by_group": {"what": "timed steps: a launch per stencil group, small groups in runs",
+                                 "launches_per_substep": ctx.num_launches(),
+                                 "projection_ms_per_substep": st["projection_ms"] / nsub,
+                                 "roofline": {"bound": "hbm", "kernel": f"xpbdProjectKernel<{dom}>",
+                                              "achieved": per_type[dom]["achieved_GBs"], "peak": HBM_PEAK_GBS,
+                                              "unit": "GB/s", "frac": per_type[dom]["frac"]},
+                                 "per_type": per_type},
+           "fp64_solves": st["fp64_solves"], "setup_s": setup, "state_finite": finite}
     if not args.no_cpu:
         out["cpu_baseline"] = xpbd_cpu_baseline(scene)
     return out
@@ -509,8 +555,13 @@ def implicit_throughput(scene, args):
     spmv_ms = tst["spmv_sampled_ms"] / max(1, tst["spmv_sampled"])
     b2b_ms = ctx.bench_spmv(1.0, -scene.dt ** 2, repeats=50)
     bytes_spmv = ctx.spmv_bytes()
-    achieved = bytes_spmv / (spmv_ms * 1e-3) / 1e9
     dofs = ctx.num_dofs()
+    # small systems (product and six vectors below 192 MB) take an iteration in two kernels, the first of which also reads p
+    # and q and writes both: 72 bytes a row more than the product's x and y
+    two_kernels = bytes_spmv + 48 * dofs < 201326592
+    if two_kernels:
+        bytes_spmv += 24 * dofs
+    achieved = bytes_spmv / (spmv_ms * 1e-3) / 1e9
     iters = st["cg_iterations"] / steps
     converged = st["last_cg_error"] <= 1e-5
     status = ("CG converged" if converged else
@@ -524,10 +575,11 @@ def implicit_throughput(scene, args):
            "last_cg_error": st["last_cg_error"], "assembly_ms_per_step": tst["assembly_ms"] / timing_steps,
            "cg_ms_per_step": tst["cg_ms"] / timing_steps,
            "cg_us_per_iteration": tst["cg_ms"] * 1e3 / max(1, tst["cg_iterations"]),
-           "roofline": {"bound": "hbm", "kernel": "cgProductKernel", "achieved": achieved, "peak": HBM_PEAK_GBS,
-                        "unit": "GB/s", "frac": achieved / HBM_PEAK_GBS, "mean_launch_us": spmv_ms * 1e3,
-                        "sampled_launches": tst["spmv_sampled"], "algorithmic_bytes_per_launch": bytes_spmv,
-                        "back_to_back_launch_us": b2b_ms * 1e3},
+           "roofline": {"bound": "hbm", "kernel": "cgProductKernel" if two_kernels else "symSpmvKernel",
+                        "achieved": achieved, "peak": HBM_PEAK_GBS, "unit": "GB/s", "frac": achieved / HBM_PEAK_GBS,
+                        "mean_launch_us": spmv_ms * 1e3, "sampled_launches": tst["spmv_sampled"],
+                        "algorithmic_bytes_per_launch": bytes_spmv,
+                        "back_to_back": {"kernel": "symSpmvKernel", "launch_us": b2b_ms * 1e3}},
            "setup_s": setup, "state_finite": finite}
     if not args.no_cpu:
         out["cpu_baseline"] = implicit_cpu_baseline()
