@@ -25,7 +25,11 @@ constexpr double kTileLaunchUs = 5.0;     // a tile launch without its groups
 constexpr double kBytesPerUs = 5e6;       // record streaming and particle gathers of a tile launch
 constexpr double kParticleBytes = 64;     // of a particle that a tile loads
 constexpr int kComputeUnits = 256;
-constexpr int kPlanThreads = 8;           // host threads that build the plan
+
+// Host threads that build the plan. Starting them takes 0.5 ms, more than the whole plan of a small mesh: 0.07 ms for a cloth
+// of 16x16 particles in 20 groups.
+constexpr int kPlanThreads = 8;
+constexpr int64_t kThreadedFrom = 16384;  // particles times groups
 
 // A round of one group in a tile: steps of one launch of one round a group (a 100x100 cloth of each kind, solids of 12^3
 // and 17^3 cells) less the launch, by group.
@@ -142,9 +146,9 @@ std::array<Tiles, 3> makeTiles(const float *xyz, int stride, const std::vector<i
 // The stencil of a group that holds a particle: at most one does.
 class Holders {
   public:
-    Holders(int64_t nv, const std::vector<TileGroup> &groups) : m_nv(nv), m_of(nv * groups.size())
+    Holders(int64_t nv, const std::vector<TileGroup> &groups, int hostThreads) : m_nv(nv), m_of(nv * groups.size())
     {
-        forAll(groups.size(), kPlanThreads, [&](int64_t g) {
+        forAll(groups.size(), hostThreads, [&](int64_t g) {
             int32_t *of = m_of.data() + g * nv;
             std::fill(of, of + nv, -1);
             for (int32_t s = 0; s < groups[g].count; ++s)
@@ -278,7 +282,7 @@ std::vector<TileBatch> cut(const Tiles &tiles, const Holders &holders, const std
 
 // Fills the plan's lists for its batches. Returns false where a tile that was not sampled needs more particles than a
 // tile may load, or the lists outgrow their indices.
-bool fill(TilePlan &plan, const Tiles &tiles, const Holders &holders, const std::vector<TileGroup> &groups)
+bool fill(TilePlan &plan, const Tiles &tiles, const Holders &holders, const std::vector<TileGroup> &groups, int hostThreads)
 {
     struct Built {
         std::vector<int32_t> particles;
@@ -292,7 +296,7 @@ bool fill(TilePlan &plan, const Tiles &tiles, const Holders &holders, const std:
         std::vector<Built> built(nt);
         std::atomic<bool> ok{true};
         const int64_t chunk = std::max<int64_t>(1, nt / (8 * kPlanThreads));
-        forAll((nt + chunk - 1) / chunk, kPlanThreads, [&](int64_t c) {
+        forAll((nt + chunk - 1) / chunk, hostThreads, [&](int64_t c) {
             Grower grower(holders, groups);
             std::vector<std::vector<int32_t>> stencils(batch.groups);
             for (int64_t t = c * chunk; t < std::min(nt, (c + 1) * chunk) && ok; ++t) {
@@ -345,7 +349,7 @@ bool fill(TilePlan &plan, const Tiles &tiles, const Holders &holders, const std:
         }
         plan.particles.resize(particleAt[nt]);
         plan.entries.resize(entryAt[nt]);
-        forAll(nt, kPlanThreads, [&](int64_t t) {
+        forAll(nt, hostThreads, [&](int64_t t) {
             std::copy(built[t].particles.begin(), built[t].particles.end(), plan.particles.begin() + particleAt[t]);
             std::copy(built[t].entries.begin(), built[t].entries.end(), plan.entries.begin() + entryAt[t]);
         });
@@ -373,18 +377,19 @@ TilePlan buildTilePlan(const float *xyz, int stride, const std::vector<int64_t> 
         any |= waves(fewest) * groupUs(g.type) < aloneUs(g);
     }
     if (!any) return {};
+    const int hostThreads = nv * static_cast<int64_t>(groups.size()) < kThreadedFrom ? 1 : kPlanThreads;
     std::vector<std::vector<int32_t>> stencilsOf(groups.size());
-    forAll(groups.size(), kPlanThreads, [&](int64_t g) {
+    forAll(groups.size(), hostThreads, [&](int64_t g) {
         stencilsOf[g].resize(static_cast<size_t>(groups[g].count) * groups[g].size);
         stencils(static_cast<int32_t>(g), stencilsOf[g].data());
         groups[g].stencils = stencilsOf[g].data();
     });
-    const Holders holders(nv, groups);
+    const Holders holders(nv, groups, hostThreads);
     auto tiles = makeTiles(xyz, stride, objects);
     for (double margin : {1.125, 1.5, 2.0}) {
         std::array<std::vector<TileBatch>, 3> batches;
         std::array<double, 3> us;
-        forAll(3, kPlanThreads, [&](int64_t k) {
+        forAll(3, hostThreads, [&](int64_t k) {
             if (k > 0 && tiles[k].count() == tiles[k - 1].count()) {  // small objects: the same tiles
                 us[k] = std::numeric_limits<double>::max();
                 return;
@@ -406,7 +411,7 @@ TilePlan buildTilePlan(const float *xyz, int stride, const std::vector<int64_t> 
         }
         TilePlan plan;
         plan.batches = std::move(batches[best]);
-        if (fill(plan, t, holders, groups)) return plan;
+        if (fill(plan, t, holders, groups, hostThreads)) return plan;
     }
     return {};
 }
