@@ -27,10 +27,11 @@ __device__ __forceinline__ void countFp64(bool fell, unsigned long long *counter
 }
 
 // The projection of one stencil of each type (xpbd.cpp:84-95) on the positions `pos` of the particles i0 .. i3: global
-// memory, or a tile's LDS. s: 1 / dt^2. `counters` (null: not counted) receives whether it was solved in FP64, ahead of the
-// stores: the records are then written whole, where the compiler would otherwise leave out their unchanged fourth value,
-// and scattered 12-byte stores cost more than 16-byte ones (a substep with a launch per group, the count after and ahead of
-// the stores, us: 1024x1024 cloth 196 and 192, 80^3-cell solid 206 and 201, 700x700 cloth with continuum springs 256 and 251).
+// memory, or a tile's LDS. s: 1 / dt^2. `counters` receives whether it was solved in FP64, if it `counts` (the address is the
+// same in every lane: a wavefront adds once), ahead of the stores: the records are then written whole, where the compiler
+// would otherwise leave out their unchanged fourth value, and scattered 12-byte stores cost more than 16-byte ones (a
+// substep with a launch per group, the count after and ahead of the stores, us: 1024x1024 cloth 196 and 192, 80^3-cell
+// solid 206 and 201, 700x700 cloth with continuum springs 256 and 251).
 template <class P>
 __device__ __forceinline__ void projectSpring(P pos, int32_t i0, int32_t i1, float L0, float c, float s)
 {
@@ -50,13 +51,13 @@ __device__ __forceinline__ void projectAnchor(P pos, int32_t i0, float4 p, float
 
 template <class P>
 __device__ __forceinline__ void projectStvk(P pos, int32_t i0, int32_t i1, int32_t i2, float4 D, float4 c, float2 c2,
-                                            float s, unsigned long long *counters)
+                                            float s, unsigned long long *counters, bool counts)
 {
     const float4 X0 = pos[i0], X1 = pos[i1], X2 = pos[i2];
     V3f o0, o1, o2;
     const bool fell = xpbdStvkF(xyz(X0), xyz(X1), xyz(X2), X0.w, X1.w, X2.w, D.x, D.y, D.z, D.w, c.x * s, c.y * s,
                                 c.z * s, c.w * s, c2.x * s, c2.y * s, o0, o1, o2);
-    countFp64(fell, counters);
+    countFp64(fell && counts, counters);
     pos[i0] = moved(X0, o0);
     pos[i1] = moved(X1, o1);
     pos[i2] = moved(X2, o2);
@@ -78,14 +79,14 @@ __device__ __forceinline__ void projectBending(P pos, int32_t i0, int32_t i1, in
 // d2: D22 and the compliances c00, c01, c11
 template <class P>
 __device__ __forceinline__ void projectSnh(P pos, int32_t i0, int32_t i1, int32_t i2, int32_t i3, float4 d0, float4 d1,
-                                           float4 d2, float hyd, float s, unsigned long long *counters)
+                                           float4 d2, float hyd, float s, unsigned long long *counters, bool counts)
 {
     const float D[9] = {d0.x, d0.y, d0.z, d0.w, d1.x, d1.y, d1.z, d1.w, d2.x};
     const float4 X0 = pos[i0], X1 = pos[i1], X2 = pos[i2], X3 = pos[i3];
     V3f o0, o1, o2, o3;
     const bool fell = xpbdSnhF(xyz(X0), xyz(X1), xyz(X2), xyz(X3), X0.w, X1.w, X2.w, X3.w, D, d2.y * s, d2.z * s,
                                d2.w * s, hyd, o0, o1, o2, o3);
-    countFp64(fell, counters);
+    countFp64(fell && counts, counters);
     pos[i0] = moved(X0, o0);
     pos[i1] = moved(X1, o1);
     pos[i2] = moved(X2, o2);
@@ -94,7 +95,7 @@ __device__ __forceinline__ void projectSnh(P pos, int32_t i0, int32_t i1, int32_
 
 template <int T, class P>
 __device__ __forceinline__ void projectFurther(P pos, const int32_t (&vv)[4], const float4 (&c)[3], float s,
-                                               unsigned long long *counters)
+                                               unsigned long long *counters, bool counts)
 {
     constexpr int NS = xpbdFurtherStencil(T);
     float4 X[4];
@@ -115,7 +116,7 @@ __device__ __forceinline__ void projectFurther(P pos, const int32_t (&vv)[4], co
         ps[4 * q + 3] = c[q].w;
     }
     const bool fell = xpbdFurtherRecord<true>(T, xs, ws, ps, s, dx);
-    countFp64(fell, counters);
+    countFp64(fell && counts, counters);
 #pragma unroll
     for (int k = 0; k < NS; ++k)
         pos[vv[k]] = moved(X[k], V3f{float(dx[3 * k]), float(dx[3 * k + 1]), float(dx[3 * k + 2])});
@@ -134,20 +135,20 @@ __device__ __forceinline__ void projectStencil(const XpbdArgs &a, int32_t i)
         projectAnchor(a.pos, id, a.ancP[i], a.invdt2);
     } else if constexpr (T == kStvk) {
         const int4 id = a.triI[i];
-        projectStvk(a.pos, id.x, id.y, id.z, a.triD[i], a.triC0[i], a.triC1[i], a.invdt2, a.counters);
+        projectStvk(a.pos, id.x, id.y, id.z, a.triD[i], a.triC0[i], a.triC1[i], a.invdt2, a.counters, true);
     } else if constexpr (T == kBending) {
         const int4 id = a.hinI[i];
         const float2 p = a.hinP[i];
         projectBending(a.pos, id.x, id.y, id.z, id.w, p.x, p.y, a.invdt2);
     } else if constexpr (T == kSnh) {
         const int4 id = a.tetI[i];
-        projectSnh(a.pos, id.x, id.y, id.z, id.w, a.tetD0[i], a.tetD1[i], a.tetD2[i], a.tetH[i], a.invdt2, a.counters);
+        projectSnh(a.pos, id.x, id.y, id.z, id.w, a.tetD0[i], a.tetD1[i], a.tetD2[i], a.tetH[i], a.invdt2, a.counters, true);
     } else if constexpr (T >= 6) {
         const int4 id = a.extI[i];
         const int64_t q = 3 * static_cast<int64_t>(i);
         const int32_t vv[4] = {id.x, id.y, id.z, id.w};
         const float4 c[3] = {a.extP[q], a.extP[q + 1], a.extP[q + 2]};
-        projectFurther<T>(a.pos, vv, c, a.invdt2, a.counters);
+        projectFurther<T>(a.pos, vv, c, a.invdt2, a.counters, true);
     }
 }
 
@@ -226,21 +227,21 @@ __device__ __forceinline__ void projectTileRecord(float4 *pos, const float4 (&r)
 {
     const uint32_t lo = __float_as_uint(r[0].x), hi = __float_as_uint(r[0].y);
     const int32_t i0 = lo & 0x7fff, i1 = lo >> 16, i2 = hi & 0xffff, i3 = hi >> 16;
-    if (!(lo & kTileCounts)) counters = nullptr;  // another tile counts it
+    const bool counts = lo & kTileCounts;  // else another tile counts it
     if constexpr (T == kSpring)
         projectSpring(pos, i0, i1, r[0].z, r[0].w, s);
     else if constexpr (T == kAnchor)
         projectAnchor(pos, i0, r[1], s);
     else if constexpr (T == kStvk)
-        projectStvk(pos, i0, i1, i2, r[1], r[2], make_float2(r[0].z, r[0].w), s, counters);
+        projectStvk(pos, i0, i1, i2, r[1], r[2], make_float2(r[0].z, r[0].w), s, counters, counts);
     else if constexpr (T == kBending)
         projectBending(pos, i0, i1, i2, i3, r[0].z, r[0].w, s);
     else if constexpr (T == kSnh)
-        projectSnh(pos, i0, i1, i2, i3, r[1], r[2], r[3], r[0].z, s, counters);
+        projectSnh(pos, i0, i1, i2, i3, r[1], r[2], r[3], r[0].z, s, counters, counts);
     else {
         const int32_t vv[4] = {i0, i1, i2, i3};
         const float4 c[3] = {r[1], r[2], r[3]};
-        projectFurther<T>(pos, vv, c, s, counters);
+        projectFurther<T>(pos, vv, c, s, counters, counts);
     }
 }
 
