@@ -62,7 +62,9 @@ typedef struct {
                                    column per lower block, 24 B of x and 24 B of y per block row, 16 B of
                                    row pointers per block row */
     double spmv_sampled_ms;     /* HIP-event time of the sampled SpMVs inside timed solves (the first of
-                                   every chunk of 8 iterations) */
+                                   every chunk of 8 iterations). In systems below 192 MB of product and
+                                   vectors the launch also ends the iteration before and updates p and q,
+                                   72 B a block row beside spmv_bytes */
     int64_t spmv_sampled;       /* how many were sampled */
 } spg_implicit_stats;
 

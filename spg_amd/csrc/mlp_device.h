@@ -1,4 +1,4 @@
-// Device-side interface of the learned warm start: network shape, GEMM epilogue and kernel launchers.
+// Device-side interface of the learned warm start: network shape and kernel launchers.
 #pragma once
 
 #include <hip/hip_runtime.h>

@@ -211,9 +211,10 @@ __global__ void __launch_bounds__(256) mlpInferKernel(const float *__restrict__ 
 // rows as K. Its sums over the row blocks it takes go to its own part of `partial`; mlpUpdateKernel adds the parts up in
 // a fixed order.
 //
-// What bounds it: latency. A minibatch of 4096 rows is 64 workgroups of about 400 MFMAs a wavefront; as separate
-// products (eleven of them, and 12 further launches) it took 420 us, most of it the weight gradients' serial K loop over
-// the batch in four workgroups. Now it is this kernel, 24 us, and mlpUpdateKernel, 7 us.
+// What bounds it: latency. A minibatch of 4096 rows is 64 workgroups of one wavefront a SIMD, each with 224 MFMAs a row block
+// (148 forward and back, 76 for its part of the weight gradients) and 2,800 vector instructions in a chain: a quarter of its
+// cycles issue one. As separate products (eleven of them, and 12 further launches) a minibatch took 420 us, most of it the
+// weight gradients' serial K loop over the batch in four workgroups. Now it is this kernel, 24 us, and mlpUpdateKernel, 7 us.
 constexpr int kTrainRows = 64;
 constexpr int kRowStride = kTrainRows + 8;  // bf16 per LDS feature row: 16-byte aligned, no bank conflicts
 constexpr int kSplit = 4;                   // threads that share a parameter's partial sums in mlpUpdateKernel

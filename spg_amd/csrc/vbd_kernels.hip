@@ -144,7 +144,8 @@ __device__ __forceinline__ int blockSolve(const S3f &H, const V3f &f, V3f &dx)
         const double d11 = xx * zz - xz * xz, d12 = xy * xz - xx * yz, d22 = xx * yy - xy * xy;
         const double fx = f.x, fy = f.y, fz = f.z;
         // one FP64 division instead of three (each some ten instructions, of the 708 of a wavefront whose launch they
-        // bound: twenty sweeps of a flat 512x512 cloth 884 -> 854 us); the rounding to FP32 hides the difference
+        // bound: twenty sweeps of a flat 512x512 cloth 884 -> 854 us). The quotients differ by an ulp or two of FP64, which
+        // the rounding to FP32 lets through once in some 10^8; that cloth's state is the same bit for bit (6 and 8 lanes)
         const double id = 1.0 / det64;
         dx.x = static_cast<float>((d00 * fx + d01 * fy + d02 * fz) * id);
         dx.y = static_cast<float>((d01 * fx + d11 * fy + d12 * fz) * id);

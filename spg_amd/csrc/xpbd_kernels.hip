@@ -252,8 +252,12 @@ __device__ __forceinline__ void projectTileRecord(float4 *pos, const float4 (&r)
 //
 // What bounds it: the chain of groups, about 1 us each (LDS reads, 300 to 400 dependent instructions, barrier), in which
 // a thread has one stencil. Hence as many threads as the registers allow on tiles of 256 to 1024 particles: the halo's
-// stencils fill threads that would be idle. One launch a substep instead of 20 on a 512x512 cloth: 89 us a substep with
-// a launch per group (small ones in runs), 30 us in tiles; 17^3-cell cube 128 us and 59 us; 32x32 cloth 80 and 19 us.
+// stencils fill threads that would be idle. A 512x512 cloth's 256 tiles issue vector instructions in 73% of a SIMD's cycles
+// (16 wavefronts a tile, 2,700 each), of which half are for the halo (2.4 million projections for 1.3 million stencils). A
+// solid of 17^3 cells has 24 tiles for 256 compute units, which project 155,000 times for 29,800 stencils; its SIMDs issue
+// in 41% of the cycles, the rest is the latency of two wavefronts' chains, and no projection takes FP64. One launch a substep
+// instead of 20 on the cloth: 89 us a substep with a launch per group (small ones in runs), 31 us in tiles; the solid
+// (three launches) 125 us and 60 us; 32x32 cloth 80 and 19 us.
 //
 // SET: the energy types compiled in (tileSet), so that a cloth's kernel holds no registers for the FP64 solve of a
 // tetrahedron.

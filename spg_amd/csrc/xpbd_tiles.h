@@ -20,8 +20,8 @@ namespace spgvbd {
 constexpr int kTileSurface = 0, kTileFive = 1, kTileFurther = 2;
 constexpr int tileSet(int type) { return type >= 6 ? kTileFurther : type == 4 ? kTileFive : kTileSurface; }
 // Threads of a tile's workgroup. A group takes a round per this many of the tile's stencils; 1024 threads leave 128
-// registers each, too few for a tetrahedron's FP64 solve (512x512 cloth: 30 us a substep with 1024 threads, 36 with 512,
-// 44 with 256; 17^3-cell cube: 153, 59 and 78).
+// registers each, too few for a tetrahedron with its FP64 solve, whose path few projections take but whose registers all
+// hold (170; 512x512 cloth: 30 us a substep with 1024 threads, 36 with 512, 44 with 256; 17^3-cell cube: 153, 59 and 78).
 constexpr int tileThreads(int set) { return set == kTileSurface ? 1024 : 512; }
 constexpr int kTileMaxParticles = 3968;  // particles a tile loads at most: 62 KB of LDS
 constexpr int kTileMaxGroups = 64;       // groups of a batch at most
