@@ -478,11 +478,12 @@ def xpbd_throughput(scene, args):
     wall = run(nsub)
     substep_us = (run(2 * nsub) - wall) / (steps * nsub) * 1e6
     plan = ctx.substep_plan()
-    ctx.reset_stats()
     ctx.set_timing(True)
-    ctx.restore_state()
-    ctx.step(scene.dt, nsub, scene.gravity)
-    ctx.synchronize()
+    for _ in range(2):  # the first loads the kernels' code, which the steps above did not use
+        ctx.reset_stats()
+        ctx.restore_state()
+        ctx.step(scene.dt, nsub, scene.gravity)
+        ctx.synchronize()
     st = ctx.stats()
     ctx.set_timing(False)
     finite = bool(np.isfinite(ctx.state()[0]).all())
@@ -502,7 +503,7 @@ def xpbd_throughput(scene, args):
            "value": n_st * nsub * steps / wall, "unit": "stencil-projections/s",
            "ms_per_step": wall * 1e3 / steps, "steps": steps, "substeps": nsub, "stencils": n_st,
            "substep_us": substep_us, "substep_plan": plan,
-           "roofline": {"bound": "latency of the chain of stencil groups in a tile", "kernel": "xpbdTileKernel",
+           "roofline": {"bound": "vector instructions of a chain of stencil groups", "kernel": "xpbdTileKernel",
                         "achieved": achieved, "peak": HBM_PEAK_GBS, "unit": "GB/s", "frac": achieved / HBM_PEAK_GBS,
                         "algorithmic_bytes_per_substep": substep_bytes} if plan["tiled_launches"] else None,
            "launches_by_group": {"what": "timed steps: a launch per stencil group, small groups in runs",
