@@ -554,8 +554,8 @@ void buildContext(spg_rigid_ctx &c, const spg_rigid_group *groups, int32_t nGrou
             bytes += 8 + 8 * rbParams(el.type) + (el.type == kRbAnchor ? 0 : 8 * kPose);
         }
         ptr[s + 1] = static_cast<int64_t>(inc.size());
-        // read: pose, row pointers, mass, xt, omega, local inertia, Rold; written: pose, theta
-        bytes += 8 * kPose + 16 + 8 + 24 + 24 + 72 + 72 + 8 * kPose + 24;
+        // read: pose, row pointers, mass, xt, omega, local inertia, Rold; written: pose
+        bytes += 8 * kPose + 16 + 8 + 24 + 24 + 72 + 72 + 8 * kPose;
     }
     c.incEntries = static_cast<int64_t>(inc.size());
     c.solveBytes = bytes;

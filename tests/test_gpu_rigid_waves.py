@@ -46,3 +46,13 @@ def test_copies_end_where_one_scene_ends(build, counts):
             got = got.reshape(k, -1)
             assert np.abs(got - want.ravel()).max() <= 1e-10 * max(np.abs(want).max(), 1.0)
         assert many.stats()["skipped_blocks"] == 0
+
+
+def test_bytes_of_a_sweep():
+    """What a sweep has to move, from the element counts: a body's pose read and written and the rest of its state read (the
+    rotation vectors are formed at the substep's end), per entry its 8 bytes, the parameters and the other body's pose."""
+    s = scenes.rb_lattice(6)
+    n = {kind: len(st) for kind, st, _ in s.energies}
+    want = s.nb * (96 + 16 + 8 + 24 + 24 + 72 + 72 + 96) + 2 * n["rb_spring"] * (8 + 64 + 96) + n["rb_anchor"] * (8 + 56)
+    want += 2 * n["rb_alignment"] * (8 + 8 + 96)
+    assert native.RigidContext([s]).stats()["solve_bytes"] == want
